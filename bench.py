@@ -45,12 +45,12 @@ TRAFFIC_FILE = os.path.join(ROOT, "profiles", "traffic_c3_hoisted.json")
 KERNELS = {
     "dot": ("pch::ks::dot_fast<3, true, 4, 0, false>",
             "dot_fast<3, true, 4, 0, false>: key inner product of all 26 keys, a regenerated by ChaCha12"),
-    "md_ntt": ("pch::ntt::fwd_", "fwd_cols + fwd_rows<epilogue 1>: ModDown NTT, (x - conv) P^-1"),
-    "md_intt": ("pch::ntt::inv_", "inv_rows + inv_cols: ModDown INTT of the P rows"),
+    "md_ntt": ("pch::ntt::mf_fwd_", "mf_fwd_rows<epilogue 1>: ModDown NTT row pass, (x - conv) P^-1"),
+    "md_intt": ("pch::ntt::mf_inv_", "mf_inv_rows + mf_inv_cols: ModDown INTT of the P rows"),
     "md_bconv": ("pch::bconv::bconv_k", "bconv_k: ModDown P -> Q conversion"),
-    "modup_intt": ("pch::ntt::inv_", "inv_rows + inv_cols: ModUp INTT"),
+    "modup_intt": ("pch::ntt::mf_inv_", "mf_inv_rows + mf_inv_cols: ModUp INTT"),
     "modup_bconv": ("pch::bconv::bconv_k", "bconv_k: ModUp conversion"),
-    "modup_ntt": ("pch::ntt::fwd_", "fwd_cols + fwd_rows: ModUp NTT"),
+    "modup_ntt": ("pch::ntt::mf_fwd_", "mf_fwd_rows: ModUp NTT row pass"),
 }
 
 

@@ -18,6 +18,7 @@
 
 #include "pc_hip.h"
 #include "fused.h"
+#include "mf.h"
 
 typedef unsigned __int128 u128;
 
@@ -278,6 +279,8 @@ struct pcx_ctx {
     int cc_tpw = 0;  // its targets per workgroup (0: from the launch's size; PCX_CC_TPW)
     int cc_ntg = 3, cc_ntgx = 2;  // targets per round of a thread's sums: fast, exact jobs (PCX_CC_NTG, PCX_CC_NTGX)
     int md_ntg = 5;           // its target rows per workgroup
+    // the matrix-core transforms' tables (can 0: a prime below their range, the butterflies of the kernel table run)
+    pch::MfTab mf = {};
     int32_t* digit_of = nullptr;
     std::vector<Level> levels;
     uint32_t *coef = nullptr, *digits = nullptr, *ext = nullptr, *conv = nullptr;
@@ -655,6 +658,22 @@ NttArgs ntt_args(const pcx_ctx* c, void* base, const Rows& r, int nrows) {
     return a;
 }
 
+// The transforms: on the matrix cores (mf.h), or through the kernel table's butterflies where a caller asks for the
+// table alone, for the one-pass form, or where the context's primes are below the matrix passes' range
+bool mf_on(const pcx_ctx* c) { return c->mf.can > 0 && !c->table_only; }
+int nt_fwd(const pcx_ctx* c, const NttArgs* a, pc_stream_t s) {
+    if (!mf_on(c) || pch::ntt_one_pass((int)c->logn, a->nrows)) return c->tab->ntt_fwd(a, s);
+    return pch::mf_ntt_fwd((int)c->logn, a, &c->mf, s);
+}
+int nt_inv(const pcx_ctx* c, const NttArgs* a, pc_stream_t s) {
+    if (!mf_on(c) || pch::ntt_one_pass((int)c->logn, a->nrows)) return c->tab->ntt_inv(a, s);
+    return pch::mf_ntt_inv((int)c->logn, a, &c->mf, s);
+}
+int nt_fwd_rows(const pcx_ctx* c, const NttArgs* a, pc_stream_t s) {
+    if (!mf_on(c)) return pch::ntt_fwd_rows_only((int)c->logn, a, s);
+    return pch::mf_ntt_fwd_rows((int)c->logn, a, &c->mf, s);
+}
+
 const Level* level(const pcx_ctx* c, int top) {
     if (top < 0 || top >= c->nq) return nullptr;
     return &c->levels[top];
@@ -693,7 +712,7 @@ int conv_then_rows(pcx_ctx* c, const BconvArgs& b, const NttArgs& f, pc_stream_t
         if (int e = pch::conv_cols((int)c->logn, &b, c->fw, c->fws, c->lazy, exact, ntg, tpw, s)) return e;
     }
     Stage st(c, st_rows, s);
-    return pch::ntt_fwd_rows_only((int)c->logn, &f, s);
+    return nt_fwd_rows(c, &f, s);
 }
 
 // ModUp (crates/pc-gpu/src/ks.rs:958-1040): INTT of c1 rows 0..top (out of place, N^-1 pre_t), conversion of every
@@ -724,7 +743,7 @@ int moddown_rescale(pcx_ctx* c, void* ext, int top, void* out, const void* onto,
     }
     {
         Stage st(c, 4, s);
-        if (int e = c->tab->ntt_inv(&a, s)) return e;
+        if (int e = nt_inv(c, &a, s)) return e;
     }
     BconvArgs b;
     memset(&b, 0, sizeof b);
@@ -750,7 +769,7 @@ int moddown_rescale(pcx_ctx* c, void* ext, int top, void* out, const void* onto,
         if (int e = c->tab->bconv(&b, s)) return e;
     }
     Stage st(c, 6, s);
-    return c->tab->ntt_fwd(&f, s);
+    return nt_fwd(c, &f, s);
 }
 // K <= k_max consecutive ciphertexts (ct_words apart): digits of ciphertext k at digits + k dnum rows N
 int modup(pcx_ctx* c, const void* ct, int top, pc_stream_t s, int K = 1) {
@@ -764,7 +783,7 @@ int modup(pcx_ctx* c, const void* ct, int top, pc_stream_t s, int K = 1) {
     a.ess = L->mu_intt.es + L->mu_intt.n;
     {
         Stage st(c, 0, s);
-        if (int e = c->tab->ntt_inv(&a, s)) return e;
+        if (int e = nt_inv(c, &a, s)) return e;
     }
     BconvArgs b;
     memset(&b, 0, sizeof b);
@@ -782,7 +801,7 @@ int modup(pcx_ctx* c, const void* ct, int top, pc_stream_t s, int K = 1) {
         if (int e = c->tab->bconv(&b, s)) return e;
     }
     Stage st(c, 2, s);
-    return c->tab->ntt_fwd(&f, s);
+    return nt_fwd(c, &f, s);
 }
 
 // the dot of keys [r0, r0 + m) of k into m extended ciphertexts at ext (crates/pc-gpu/src/ks.rs:1225-1308 dot_key);
@@ -915,7 +934,7 @@ int moddown(pcx_ctx* c, void* ext, uint32_t* conv, int m, int top, void* out, pc
     }
     {
         Stage st(c, 4, s);
-        if (int e = c->tab->ntt_inv(&a, s)) return e;
+        if (int e = nt_inv(c, &a, s)) return e;
     }
     const Rows& rn = L->md_ntt[m - 1];
     NttArgs f = ntt_args(c, conv, rn, rn.n);
@@ -948,7 +967,7 @@ int moddown(pcx_ctx* c, void* ext, uint32_t* conv, int m, int top, void* out, pc
             if (int e = pch::md_conv_cols((int)c->logn, &d, s)) return e;
         }
         Stage st(c, 6, s);
-        return pch::ntt_fwd_rows_only((int)c->logn, &f, s);
+        return nt_fwd_rows(c, &f, s);
     }
     BconvArgs b;
     memset(&b, 0, sizeof b);
@@ -965,7 +984,7 @@ int moddown(pcx_ctx* c, void* ext, uint32_t* conv, int m, int top, void* out, pc
         if (int e = c->tab->bconv(&b, s)) return e;
     }
     Stage st(c, 6, s);
-    return c->tab->ntt_fwd(&f, s);
+    return nt_fwd(c, &f, s);
 }
 
 // out = a + b on Q rows 0..top of both parts (the table's ew_add)
@@ -1181,6 +1200,21 @@ pcx_ctx* pcx_ctx_new_k(uint32_t log_n, const uint64_t* primes, int nq, int kp, i
     c->iws = c->dev.upload(iws);
     c->ninv = c->dev.upload(ninv);
     c->ninvs = c->dev.upload(ninvs);
+    // the matrix-core transforms' tables: the matrices per prime, the twiddle powers by a kernel from fw / iw
+    c->mf.can = pch::mf_can(c->primes.data(), R);
+    if (c->mf.can && !c->dev.err) {
+        std::vector<uint32_t> mat((size_t)R * pch::MF_MATS * 1024), ini((size_t)R * pch::MF_MATS * 64);
+        for (int id = 0; id < R; ++id)
+            pch::mf_build_mats((int)log_n, c->primes[id], c->roots[id], &mat[(size_t)id * pch::MF_MATS * 1024],
+                               &ini[(size_t)id * pch::MF_MATS * 64]);
+        c->mf.mat = c->dev.upload(mat);
+        c->mf.init = c->dev.upload(ini);
+        const size_t tw = (size_t)R * pch::mf_tw_words((int)log_n) * 4;
+        uint32_t *f = (uint32_t*)c->dev.alloc(tw), *v = (uint32_t*)c->dev.alloc(tw);
+        c->mf.tw = f;
+        c->mf.itw = v;
+        if (!c->dev.err) c->dev.err = pch::mf_build_tw((int)log_n, R, c->fw, c->iw, c->pr, f, v, nullptr);
+    }
     // P mod q and P^-1 mod q by prime id, then their Shoup companions (crates/pc-gpu/src/context.rs:234-259)
     std::vector<uint32_t> pm(R, 0), pi(R, 0);
     for (int t = 0; t < nq; ++t) {
@@ -1345,7 +1379,7 @@ int pcx_ntt_one_pass_min(int rows) { return pch::ntt_one_pass_min(rows); }
 int pcx_ntt(pcx_ctx* c, int dir, void* base, const pcx_rows* rows, pc_stream_t s) {
     if (!c || !rows || (dir != 1 && dir != -1)) return -1;
     NttArgs a = ntt_args(c, base, rows->r, rows->r.n);
-    return dir == 1 ? c->tab->ntt_fwd(&a, s) : c->tab->ntt_inv(&a, s);
+    return dir == 1 ? nt_fwd(c, &a, s) : nt_inv(c, &a, s);
 }
 
 // A key group from host b ([ndig][srows][N] per key, dense words) and seeds, banded at q_top (nq - 1: full rows)
@@ -1448,7 +1482,7 @@ static pcx_keys* keys_generate(pcx_ctx* c, int nkeys, const uint64_t* galois, co
         return nullptr;
     }
     NttArgs a = ntt_args(c, s_eval, rows_all, R);
-    int rc = c->tab->ntt_fwd(&a, s);
+    int rc = nt_fwd(c, &a, s);
     std::vector<const void*> kb;
     std::vector<const uint32_t*> sd;
     for (int r = 0; r < nkeys && !rc; ++r) {
@@ -1469,7 +1503,7 @@ static pcx_keys* keys_generate(pcx_ctx* c, int nkeys, const uint64_t* galois, co
             break;
         }
         NttArgs ea = ntt_args(c, e, rows_e, c->dnum * R);
-        if ((rc = c->tab->ntt_fwd(&ea, s))) break;
+        if ((rc = nt_fwd(c, &ea, s))) break;
         AutomorphArgs au;
         memset(&au, 0, sizeof au);
         au.out = PolyRef{s_new, 0, 0};
@@ -1972,7 +2006,7 @@ int pcx_rescale_k(pcx_ctx* c, const void* ct, int top, int ndrop, void* out, int
     if (ct != out)
         if (int e = copy_q(c, ct, top, out, s, K)) return e;
     NttArgs in = ntt_args(c, out, Z.intt, k_rows(c, Z.intt, K));
-    if (int e = c->tab->ntt_inv(&in, s)) return e;
+    if (int e = nt_inv(c, &in, s)) return e;
     RescaleArgs r;
     memset(&r, 0, sizeof r);
     const uint64_t part = (uint64_t)R * c->n;
@@ -2003,10 +2037,10 @@ int pcx_rescale_k(pcx_ctx* c, const void* ct, int top, int ndrop, void* out, int
         RescaleNttArgs a;
         a.rs = r;
         a.ntt = f;
-        return c->tab->rescale_fwd(&a, s);
+        return mf_on(c) ? pch::mf_rescale_fwd((int)c->logn, &a, &c->mf, s) : c->tab->rescale_fwd(&a, s);
     }
     if (int e = c->tab->rescale_coef(&r, s)) return e;
-    return c->tab->ntt_fwd(&f, s);
+    return nt_fwd(c, &f, s);
 }
 int pcx_rescale(pcx_ctx* c, const void* ct, int top, int ndrop, void* out, pc_stream_t s) {
     return pcx_rescale_k(c, ct, top, ndrop, out, 1, s);
@@ -2293,7 +2327,7 @@ int pcx_decrypt_rows(pcx_decryptor* x, const void* ct, int K, int top, int which
     if (int e = c->tab->tensor(&t, s)) return e;
     const Rows& r = x->lists[K - 1];
     NttArgs a = ntt_args(c, x->out, r, r.n);
-    if (int e = c->tab->ntt_inv(&a, s)) return e;
+    if (int e = nt_inv(c, &a, s)) return e;
     for (int cc = 0; cc < K; ++cc) {
         hipError_t e = hipMemcpyAsync((uint32_t*)out + cc * dn, x->out + cc * 2 * dn + dn, dn * sizeof(uint32_t),
                                       hipMemcpyDeviceToDevice, (hipStream_t)s);

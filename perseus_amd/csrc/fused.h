@@ -80,6 +80,8 @@ void ntt1_inv(const NttArgs& a, int r0, int n, pc_stream_t st);
 int ntt_fwd_dense(int logn, const NttArgs* a, pc_stream_t s);
 // the row count from which launches of N = 2^16 take the one-pass transform (0: never); returns the previous one
 int ntt_one_pass_min(int rows);
+// whether a launch of that many rows takes it
+bool ntt_one_pass(int logn, int rows);
 
 // noalloc.hip: looks up the no-allocation ladder's scratch address on the current device (0 or the HIP error)
 int noalloc_prepare();

@@ -28,38 +28,6 @@ namespace pch {
 namespace ntt {
 
 // ------------------------------------------------------------------------------------------------ forward
-// The composite rescale's correction row (rescale_fwd, args.cuh RescaleArgs / RescaleNttArgs :531-563), generated in
-// the column pass instead of loaded: row i of the transform is tmp row r = rprime[i] of its polynomial, whose two
-// sources sit top - r and top - 1 - r rows above it (y_a scaled by ca, and y' = (y_b - lift(y_a)) / q_a mod q_b, both
-// canonical): x = A_r lift(y_a) + B_r lift(y'), lift(y) = y - q_top (q_top - 1) when y > q_top / 2 (q_top-1 / 2),
-// reduced mod q_r.
-struct RsGen {
-    const uint32_t* ya;
-    const uint32_t* yp;
-    uint32_t q, m, ha, hb, av, as, bv, bs, qam, qbm;
-    __device__ __forceinline__ RsGen(const RescaleArgs& R, const uint32_t* row, int r, int logn) {
-        ya = row + ((size_t)(R.top - r) << logn);
-        yp = row + ((size_t)(R.top - 1 - r) << logn);
-        q = (uint32_t)R.pr[r].p;
-        m = (uint32_t)(R.pr[r].mu_lo >> 32);
-        ha = (uint32_t)R.pr[R.top].p >> 1;
-        hb = (uint32_t)R.pr[R.top - 1].p >> 1;
-        av = ((const uint32_t*)R.A)[r];
-        as = ((const uint32_t*)R.As)[r];
-        bv = ((const uint32_t*)R.B)[r];
-        bs = ((const uint32_t*)R.Bs)[r];
-        qam = ((const uint32_t*)R.qam)[r];
-        qbm = ((const uint32_t*)R.qbm)[r];
-    }
-    __device__ __forceinline__ uint32_t operator()(size_t o) const {
-        const uint32_t u = ya[o], v = yp[o];
-        uint32_t la = red32(u, q, m), lb = red32(v, q, m);
-        if (u > ha) la = subm(la, qam, q);
-        if (v > hb) lb = subm(lb, qbm, q);
-        return addm(shoup(la, av, as, q), shoup(lb, bv, bs, q), q);
-    }
-};
-
 // Column pass: workgroup (x, row i) takes columns [x CC, x CC + CC) of row i. GEN: the rows are rescale corrections
 // generated by RsGen from R.
 template <int LOGN, bool H, bool GEN = false>
@@ -455,6 +423,7 @@ int fwd_dense(const NttArgs* a, pc_stream_t s) {
 }
 }  // namespace ntt
 
+bool ntt_one_pass(int logn, int rows) { return ntt::one_pass(logn, rows); }
 int ntt_one_pass_min(int rows) {
     const int prev = ntt::ntt1_min();
     ntt::g_ntt1_min.store(rows < 0 ? 0 : rows, std::memory_order_relaxed);

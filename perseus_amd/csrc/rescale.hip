@@ -11,6 +11,7 @@
 // rescale_fwd: the correction rows are never stored: a prep kernel writes the two sources of every coefficient (y_a,
 // y') into tmp rows top and top - 1, and the forward NTT's column pass generates each correction row from them.
 #include "fused.h"
+#include "mf.h"
 #include "common.h"
 
 namespace pch {
@@ -111,8 +112,9 @@ int coef(const RescaleArgs* a, pc_stream_t s) {
     return launch_rc();
 }
 
+// mf: the transform on the matrix cores (the driver's tables), null: the butterflies
 template <int LOGN>
-int fwd(const RescaleNttArgs* a, pc_stream_t s) {
+int fwd(const RescaleNttArgs* a, pc_stream_t s, const MfTab* mf = nullptr) {
     if (!a) return -1;
     const RescaleArgs& R = a->rs;
     const NttArgs& T = a->ntt;
@@ -124,10 +126,21 @@ int fwd(const RescaleNttArgs* a, pc_stream_t s) {
     NttArgs b = T;
     b.snum = 1;
     b.xnum = T.xnum > 1 ? T.xnum : 1;
-    return ntt_fwd_rescale(LOGN, &b, &R, s);
+    return mf ? mf_ntt_fwd_rescale(LOGN, &b, &R, mf, s) : ntt_fwd_rescale(LOGN, &b, &R, s);
 }
 
 }  // namespace rs
+
+int mf_rescale_fwd(int logn, const RescaleNttArgs* a, const MfTab* t, pc_stream_t s) {
+    switch (logn) {
+        case 12: return rs::fwd<12>(a, s, t);
+        case 13: return rs::fwd<13>(a, s, t);
+        case 14: return rs::fwd<14>(a, s, t);
+        case 15: return rs::fwd<15>(a, s, t);
+        case 16: return rs::fwd<16>(a, s, t);
+        default: return -2;
+    }
+}
 
 #define PCH_RS_INST(L)                                                                                     \
     int rescale_coef_##L(const RescaleArgs* a, pc_stream_t s) { return rs::coef<L>(a, s); }               \
