@@ -146,6 +146,74 @@ struct Bconv {
     BconvJob* jobs = nullptr;
     uint32_t* pool = nullptr;
     int njobs = 0, max_tgt = 0;
+    // the same jobs on the matrix cores (mfconv.hip): sources padded to mf_ns, 0 where that form does not apply
+    uint32_t *mf_jobs = nullptr, *mf_dig = nullptr;
+    uint32_t mf_stride = 0;
+    int mf_ns = 0, mf_src = 0;  // mf_src: the most sources of a job
+
+    // logn: the rows' width. An exact job's u = round(sum y_i / b_i) is one more source, job k's in row u_row + k of src
+    void build_mf(Dev& dev, const std::vector<uint64_t>& primes, const std::vector<JobSpec>& specs, int logn,
+                  uint32_t u_row = 0) {
+        using pch::MfConvArgs;
+        size_t most = 0, tgts = 0;
+        for (const JobSpec& j : specs) {
+            most = std::max(most, j.src.size() + (j.exact ? 1 : 0));
+            mf_src = std::max(mf_src, (int)j.src.size());
+            tgts = std::max(tgts, j.tgt.size());
+        }
+        if (most < 1 || most > (size_t)pch::MFC_MAX_NS || tgts < 1) return;
+        const int ns = most <= 8 ? 8 : most <= 16 ? 16 : pch::MFC_MAX_NS;
+        const size_t stride = 8 + MfConvArgs::src_words(ns) + 8 * tgts;
+        std::vector<uint32_t> rec(specs.size() * stride, 0), dig_h, dig_at(specs.size());
+        for (size_t k = 0; k < specs.size(); ++k) {
+            const JobSpec& j = specs[k];
+            const uint32_t nt = (uint32_t)j.tgt.size();
+            std::vector<uint32_t> src = j.src;
+            if (j.exact) src.push_back(u_row + (uint32_t)k - j.src_off);
+            // ciphertexts and parts repeat a job's primes: their digits once
+            size_t same = 0;
+            while (same < k && (specs[same].src != j.src || specs[same].tgt != j.tgt || specs[same].exact != j.exact))
+                ++same;
+            dig_at[k] = same < k ? dig_at[same] : (uint32_t)dig_h.size();
+            pch::MfConvJob r = {j.src_off, j.dst_off, 1 + *std::max_element(src.begin(), src.end()),
+                                nt ? 1 + *std::max_element(j.tgt.begin(), j.tgt.end()) : 0, nt, dig_at[k], {0, 0}};
+            if (((uint64_t)std::max(r.src_rows, r.dst_rows) << (logn + 2)) >> 32) return;  // past a buffer's extent
+            uint32_t* w = &rec[k * stride];
+            memcpy(w, &r, sizeof r);
+            for (uint32_t i = 0; i < MfConvArgs::src_words(ns); ++i) w[8 + i] = src[std::min((size_t)i, src.size() - 1)];
+            for (uint32_t i = 0; i < nt; ++i) {
+                const PrimeConst pc = prime_const(primes[j.tgt[i]]);
+                const pch::MfConvTgt t = {j.tgt[i], j.tgt[i], (uint32_t)pc.p, (uint32_t)(pc.mu_lo >> 16),
+                                          (uint32_t)pc.mont_pinv, {0, 0, 0}};
+                memcpy(w + 8 + MfConvArgs::src_words(ns) + 8 * i, &t, sizeof t);
+            }
+            if (same < k) continue;
+            for (uint32_t t0 = 0; t0 < nt; t0 += 4) {
+                const uint32_t m = std::min(4u, nt - t0);
+                uint64_t p[4];
+                std::vector<uint64_t> f(src.size() * m);
+                for (uint32_t t = 0; t < m; ++t) {
+                    const uint64_t tp = p[t] = primes[j.tgt[t0 + t]];
+                    uint64_t all = 1;
+                    for (uint32_t b : j.src) all = mulmod(all, primes[b] % tp, tp);
+                    for (size_t i = 0; i < j.src.size(); ++i) {
+                        uint64_t v = 1;
+                        for (size_t x = 0; x < j.src.size(); ++x)
+                            if (x != i) v = mulmod(v, primes[j.src[x]] % tp, tp);
+                        f[i * m + t] = v;
+                    }
+                    if (j.exact) f[j.src.size() * m + t] = all ? tp - all : 0;  // less u B
+                }
+                const size_t at = dig_h.size();
+                dig_h.resize(at + MfConvArgs::group_words(ns));
+                pch::mf_conv_digits(f.data(), (int)src.size(), (int)m, p, ns, &dig_h[at]);
+            }
+        }
+        mf_jobs = dev.upload(rec);
+        mf_dig = dev.upload(dig_h);
+        mf_stride = (uint32_t)stride;
+        if (!dev.err) mf_ns = ns;
+    }
     void build(Dev& dev, const std::vector<uint64_t>& primes, const std::vector<JobSpec>& specs) {
         std::vector<uint32_t> pool_h;
         std::vector<BconvJob> jobs_h;
@@ -294,6 +362,8 @@ struct pcx_ctx {
 
     size_t row_words() const { return n; }
     size_t ct_words() const { return (size_t)2 * rows * n; }
+    // rows of the extended ciphertexts at ext; the rows after them hold the exact conversions' u, two per ciphertext
+    size_t ext_rows() const { return (size_t)std::max(k_rot, k_max) * 2 * rows; }
     int digit(int id) const { return id < nq ? id / alpha : -1; }
 };
 
@@ -456,6 +526,7 @@ int build_level(pcx_ctx* c, int top, Level& L) {
         rep_rows(roff, KM, c->dnum * RR);
         rep_rows(rp, KM, 0);
         L.mu_bconv.build(c->dev, c->primes, specs);
+        if (c->mf.can) L.mu_bconv.build_mf(c->dev, c->primes, specs, (int)c->logn);
         if (int e = fill_rows(c->dev, L.mu_ntt, roff, rp, nullptr, nullptr)) return e;
     }
     // dot rows: Q 0..top then P
@@ -482,6 +553,7 @@ int build_level(pcx_ctx* c, int top, Level& L) {
                 specs.push_back(j);
             }
         L.md_bconv.build(c->dev, c->primes, specs);
+        if (c->mf.can) L.md_bconv.build_mf(c->dev, c->primes, specs, (int)c->logn);
         L.md_intt.resize(c->k_rot);
         L.md_ntt.resize(c->k_rot);
         for (int m = 1; m <= c->k_rot; ++m) {
@@ -632,6 +704,7 @@ int build_level(pcx_ctx* c, int top, Level& L) {
         if (int e = fill_rows(c->dev, L.mdr.intt, roff, rp, nullptr, &est)) return e;
         if (int e = fill_rows(c->dev, L.mdr.ntt, roff2, rp2, nullptr, &bt)) return e;
         L.mdr.conv.build(c->dev, c->primes, specs);
+        if (c->mf.can) L.mdr.conv.build_mf(c->dev, c->primes, specs, (int)c->logn, (uint32_t)c->ext_rows());
         L.mdr.k = c->dev.upload(k);
     }
     return c->dev.err;
@@ -715,6 +788,48 @@ int conv_then_rows(pcx_ctx* c, const BconvArgs& b, const NttArgs& f, pc_stream_t
     return nt_fwd_rows(c, &f, s);
 }
 
+// Targets per workgroup: one MFMA forms four targets' words, so a run of four, two where that leaves most of the 256 CUs
+// without a workgroup (17 limbs of C3: 128 workgroups 13.9 us, at two targets 13.1; 160 workgroups 12.2 us, 13.4), two runs
+// where there are many (26 ModDowns of C3, 3328 workgroups: 205 -> 196 us; 2304: no gain). PCX_CC_TPW sets it.
+long mfc_wgs(const pcx_ctx* c, const BconvArgs& b, int t) {
+    return (long)(c->n >> (c->logn / 2)) / 16 * b.njobs * ((b.max_tgt + t - 1) / t);
+}
+int mfc_shape(const pcx_ctx* c, const BconvArgs& b) {
+    if (c->cc_tpw > 0) return c->cc_tpw > 2 ? (c->cc_tpw + 3) / 4 * 4 : c->cc_tpw;
+    return mfc_wgs(c, b, 8) >= 3000 ? 8 : mfc_wgs(c, b, 4) >= 160 ? 4 : 2;
+}
+// Above 8 sources the matrix-core form always pays (46 + 16 primes of N = 2^13, its smallest launches 384 waves: a
+// bootstrap 3098 -> 2746 us). Up to 4 the butterflies' forms sum in registers as fast (2 sources, 12 jobs of N = 2^16: a C4
+// scoring 488 against 491 us; 3 sources, 46 jobs of N = 2^12: 23 rotations 68.6 against 73.1 us). Between, it wants
+// waves to hide its chained reads and barriers: C3's ModDown of one rotation gains by it, five products of N = 2^13 (320
+// waves: 107.1 against 107.8 us) do not.
+bool mfc_on(const pcx_ctx* c, const Bconv& p, const BconvArgs& b) {
+    if (!mf_on(c) || p.mf_ns == 0) return false;
+    return c->cc_tpw > 0 || p.mf_src > 8 || (p.mf_src > 4 && mfc_wgs(c, b, 4) << (c->logn / 2) >> 5 >= 800);
+}
+// The conversion b of plan p (its first b.njobs jobs) on the matrix cores, fused into the column pass of f's rows, then f's
+// row pass and epilogue. exact: p's jobs are, b.src is the context's extended workspace
+int mfc_then_rows(pcx_ctx* c, const Bconv& p, const BconvArgs& b, const NttArgs& f, pc_stream_t s, bool exact = false) {
+    {
+        Stage st(c, exact || b.dst != c->digits ? 5 : 1, s);
+        if (exact)
+            if (int e = pch::conv_u((int)c->logn, &b, (uint32_t*)b.src + (c->ext_rows() << c->logn), s)) return e;
+        pch::MfConvArgs a;
+        a.src = (const uint32_t*)b.src;
+        a.dst = (uint32_t*)b.dst;
+        a.jobs = p.mf_jobs;
+        a.dig = p.mf_dig;
+        a.stride = p.mf_stride;
+        a.njobs = b.njobs;
+        a.max_tgt = b.max_tgt;
+        a.ns = p.mf_ns;
+        const int tpw = mfc_shape(c, b);
+        if (int e = pch::mf_conv_cols((int)c->logn, &a, &c->mf, tpw, s)) return e;
+    }
+    Stage st(c, b.dst != c->digits ? 6 : 2, s);
+    return nt_fwd_rows(c, &f, s);
+}
+
 // ModUp (crates/pc-gpu/src/ks.rs:958-1040): INTT of c1 rows 0..top (out of place, N^-1 pre_t), conversion of every
 // live digit, NTT of the targets
 // ModDown and the two-prime rescale at once (the level's mdr plan): out (Q rows 0..top - 2) = the exact
@@ -763,6 +878,7 @@ int moddown_rescale(pcx_ctx* c, void* ext, int top, void* out, const void* onto,
     f.xstride = c->ct_words();
     f.es = M.ntt.es;
     f.ess = M.ntt.es + c->rows;
+    if (mfc_on(c, M.conv, b) && c->cc_fused) return mfc_then_rows(c, M.conv, b, f, s, true);
     if (cc_on(c, CC_MDR)) return conv_then_rows(c, b, f, s, 5, 6, c->kp + 2, 1);
     {
         Stage st(c, 5, s);
@@ -795,6 +911,7 @@ int modup(pcx_ctx* c, const void* ct, int top, pc_stream_t s, int K = 1) {
     b.njobs = k_jobs(c, L->mu_bconv, K);
     b.max_tgt = L->mu_bconv.max_tgt;
     NttArgs f = ntt_args(c, c->digits, L->mu_ntt, k_rows(c, L->mu_ntt, K));
+    if (mfc_on(c, L->mu_bconv, b) && cc_on(c, CC_MODUP)) return mfc_then_rows(c, L->mu_bconv, b, f, s);
     if (cc_on(c, CC_MODUP)) return conv_then_rows(c, b, f, s, 1, 2, c->alpha);
     {
         Stage st(c, 1, s);
@@ -946,6 +1063,17 @@ int moddown(pcx_ctx* c, void* ext, uint32_t* conv, int m, int top, void* out, pc
     f.xstride = c->ct_words();
     f.es = c->pinv;
     f.ess = c->pinv + (c->nq + c->kp);
+    BconvArgs b;
+    memset(&b, 0, sizeof b);
+    b.src = ext;
+    b.dst = conv;
+    b.jobs = L->md_bconv.jobs;
+    b.pool = L->md_bconv.pool;
+    b.pr = c->pr;
+    b.njobs = 2 * m;
+    b.max_tgt = top + 1;
+    if (mfc_on(c, L->md_bconv, b) && (c->md_fused || cc_on(c, CC_MODDOWN)))
+        return mfc_then_rows(c, L->md_bconv, b, f, s);
     if (c->md_fused) {
         // the conversion inside the NTT's column pass, then the row pass with the epilogue
         pch::MdcArgs d;
@@ -969,15 +1097,6 @@ int moddown(pcx_ctx* c, void* ext, uint32_t* conv, int m, int top, void* out, pc
         Stage st(c, 6, s);
         return nt_fwd_rows(c, &f, s);
     }
-    BconvArgs b;
-    memset(&b, 0, sizeof b);
-    b.src = ext;
-    b.dst = conv;
-    b.jobs = L->md_bconv.jobs;
-    b.pool = L->md_bconv.pool;
-    b.pr = c->pr;
-    b.njobs = 2 * m;
-    b.max_tgt = top + 1;
     if (cc_on(c, CC_MODDOWN)) return conv_then_rows(c, b, f, s, 5, 6, c->kp);
     {
         Stage st(c, 5, s);
@@ -1258,10 +1377,10 @@ pcx_ctx* pcx_ctx_new_k(uint32_t log_n, const uint64_t* primes, int nq, int kp, i
     const size_t coef_rows = k_max == 1 ? (size_t)nq : (size_t)k_max * R;
     c->coef = (uint32_t*)c->dev.alloc(coef_rows * rw);
     c->digits = (uint32_t*)c->dev.alloc((size_t)k_max * dnum * R * rw);
-    c->ext = (uint32_t*)c->dev.alloc(next * 2 * R * rw);
+    c->ext = (uint32_t*)c->dev.alloc((c->ext_rows() + 2 * k_max) * rw);
     c->conv = (uint32_t*)c->dev.alloc(next * 2 * R * rw);
     c->tmp = (uint32_t*)c->dev.alloc((size_t)k_max * 2 * R * rw);
-    c->ws_bytes = (coef_rows + (size_t)k_max * dnum * R + 2 * next * 2 * R + (size_t)k_max * 2 * R) * rw;
+    c->ws_bytes = (coef_rows + (size_t)k_max * dnum * R + 2 * next * 2 * R + 2 * k_max + (size_t)k_max * 2 * R) * rw;
     if (c->dev.err) {
         *err = c->dev.err;
         delete c;

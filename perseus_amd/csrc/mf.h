@@ -51,6 +51,8 @@ constexpr uint32_t MF_FLIP = 0x80808080u;
 
 struct MfPrime {
     uint32_t p, np, mu, pinv;  // p, 2^32 - p, floor(2^48 / p), -p^-1 mod 2^32
+    __device__ __forceinline__ MfPrime(uint32_t p_, uint32_t mu_, uint32_t pinv_)
+        : p(p_), np(0u - p_), mu(mu_), pinv(pinv_) {}
     __device__ __forceinline__ MfPrime(const PrimeConst* pr, uint32_t i) {
         p = (uint32_t)sload(&pr[i].p);
         np = 0u - p;
@@ -160,6 +162,38 @@ int mf_ntt_fwd(int logn, const NttArgs* a, const MfTab* t, pc_stream_t s);
 int mf_ntt_inv(int logn, const NttArgs* a, const MfTab* t, pc_stream_t s);
 // the row pass alone, after a column pass done elsewhere
 int mf_ntt_fwd_rows(int logn, const NttArgs* a, const MfTab* t, pc_stream_t s);
+// A base-conversion plan on the matrix cores (mfconv.hip). Job k takes its source rows (src_off + a row, words prescaled;
+// every word any 32 bits) to the column pass of its targets in rows dst_off + a row.
+struct MfConvJob {
+    uint32_t src_off, dst_off;    // rows
+    uint32_t src_rows, dst_rows;  // the extents: rows read and written lie below them
+    uint32_t nt;                  // targets
+    uint32_t dig;                 // words of MfConvArgs.dig: mf_conv_digits of each four targets
+    uint32_t pad[2];
+};
+struct MfConvTgt {
+    uint32_t row, id, p, mu, pinv, pad[3];  // its row and prime id; MfPrime's constants
+};
+struct MfConvArgs {
+    const uint32_t* src;
+    uint32_t* dst;
+    const uint32_t* jobs;  // job k's words from k stride: MfConvJob, src_words(ns) source rows (past the last: any of
+    const uint32_t* dig;   // them), nt MfConvTgt
+    uint32_t stride;
+    int njobs, max_tgt, ns;  // ns: 8, 16 or 20, the jobs' sources padded
+    static constexpr __host__ __device__ uint32_t src_words(int ns) { return ((uint32_t)ns + 7) / 8 * 8; }
+    static constexpr __host__ __device__ uint32_t group_words(int ns) { return (uint32_t)ns * 16 + 16; }
+};
+constexpr int MFC_MAX_NS = 20;
+// tpw: targets per workgroup: 1, 2 or a multiple of 4. 0, -1 (bad arguments), -2 (ns or logn outside the range) or a HIP error
+int mf_conv_cols(int logn, const MfConvArgs* a, const MfTab* t, int tpw, pc_stream_t s);
+// u = floor(sum_i y_i / b_i + 1/2) of each exact job of a (bconv.hip's records: the doubles' FMAs in source order) to row k
+// of u, job k's
+int conv_u(int logn, const BconvArgs* a, uint32_t* u, pc_stream_t s);
+// host: the A operands and initial values of one run of nt <= 4 targets: w[i][t] below p[t], n sources padded to ns
+void mf_conv_digits(const uint64_t* w, int n, int nt, const uint64_t* p, int ns, uint32_t* out);
+// host: the four signed base-256 digits of w mod p, centred
+void mf_digits(uint64_t w, uint64_t p, int8_t (&d)[4]);
 // the table's rescale_fwd (rescale.hip) with its transform on the matrix cores
 int mf_rescale_fwd(int logn, const RescaleNttArgs* a, const MfTab* t, pc_stream_t s);
 // the forward transform of composite-rescale corrections (ntt_fwd_rescale)

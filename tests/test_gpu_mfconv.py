@@ -1,0 +1,82 @@
+"""The conversions on the matrix cores (mfconv.hip) against the same context's launches through the kernel table alone
+(bconv, then the transforms), word for word: one to 17 sources (padded to 8, 16 and 20, one more in the exact
+conversion), targets that leave a last run of one to four, every number of targets per workgroup that its rule chooses
+(1, 2, 4, 8: PCX_CC_TPW), every ring degree, 28- to 31-bit primes, and ciphertexts of words at the ends of their range
+(0, p - 1), where a digit sum that overflowed would show. Each test prints its case before the GPU runs."""
+import sys
+
+import numpy as np
+import pytest
+
+import perseus_amd as pa
+from perseus_amd.chains import make
+from tests import twin
+
+pytestmark = pytest.mark.gpu
+
+
+def say(*a):
+    print(*a, flush=True)
+    sys.stdout.flush()
+
+
+@pytest.fixture(scope="module")
+def stream():
+    assert pa.device_count() >= 1, "no GPU visible"
+    return pa.Stream()
+
+
+# (log N, Q primes, special primes, digits, bits, tops): sources of the ModUp ceil(nq / dnum), of the ModDown kp, of the
+# exact conversion kp + 3
+CASES = [
+    (12, 3, 1, 3, 28, [2]),
+    (12, 14, 8, 2, 31, [13, 6]),
+    (13, 9, 5, 3, 29, [8, 3]),
+    (14, 12, 4, 3, 30, [11, 10, 9]),
+    (15, 18, 9, 2, 31, [17, 8]),
+    (16, 20, 16, 3, 30, [19, 2]),
+    (12, 34, 17, 2, 30, [33]),
+]
+
+
+@pytest.mark.parametrize("logn,nq,kp,dnum,bits,tops", CASES)
+@pytest.mark.parametrize("tpw", [1, 2, 4, 8])
+def test_conversions_equal_the_tables(stream, monkeypatch, logn, nq, kp, dnum, bits, tops, tpw):
+    monkeypatch.setenv("PCX_CC_TPW", str(tpw))
+    ch = make("mfc", logn, nq, kp, dnum, bits)
+    ctx = pa.Context(ch, k_rot=2, k_max=2)
+    rng = np.random.default_rng(nq)
+    s = rng.integers(-1, 2, ch.n).astype(np.int8)
+    gals = [1, twin.rotation_galois(3, ch.n)]
+    seeds = rng.integers(0, 2**32, (2, 8), dtype=np.uint64).astype(np.uint32)
+    err = rng.integers(-3, 4, (2, ch.dnum, ch.n)).astype(np.int64)
+    keys = pa.Keys(ctx, gals, seeds=seeds, secret=s, errors=err, bits=0)
+    for top in tops:
+        for fill in ("random", "ends"):
+            ct = np.zeros((2, 2, ch.rows, ch.n), np.uint32)
+            for t in range(top + 1):
+                p = ch.primes[t]
+                ct[:, :, t] = rng.integers(0, p, (2, 2, ch.n)) if fill == "random" else p - 1
+            if fill == "ends":
+                ct[:, :, :, 1::2] = 0
+            x = pa.DevBuf.from_array(ct)
+            out = ctx.ct_buf(2)
+
+            def run(f):
+                got = []
+                for table in (False, True):
+                    ctx.table_only(table)
+                    out.zero()
+                    f()
+                    stream.sync()
+                    got.append(out.download((2, 2, ch.rows, ch.n)))
+                ctx.table_only(False)
+                return got
+
+            say(f"[mfconv] N=2^{logn} {nq}+{kp} primes of {bits} bits, top {top}, {tpw} targets, {fill}: rotations")
+            a, b = run(lambda: ctx.rotate_hoisted(keys, [0, 1], x, top, out, stream))
+            assert (a[:, :, : top + 1] == b[:, :, : top + 1]).all()
+            if top >= 2:
+                say("[mfconv]   two products, rescaled (the exact conversion)")
+                a, b = run(lambda: ctx.mul_relin_rescale(keys, x, x, top, out, stream, K=2))
+                assert (a[:, :, : top - 1] == b[:, :, : top - 1]).all()
