@@ -19,6 +19,7 @@
 //   3. to_output: the two words per slot move to output order through LDS with a conflict-free scatter (below);
 //   4. the kernel adds them into its sums (the CtS stage: times the diagonals' words at the lane's output slots).
 #include "common.h"
+#include "fused.h"
 
 namespace pch {
 namespace cts {
@@ -535,6 +536,102 @@ __global__ void __launch_bounds__(CW, 3) ksum_k(KsKeyArgs G, int logn) {
     st8(out1, acc1);
 }
 
+// KS_SUM with every digit's `a` words expanded beforehand (kska_expand: [key][digit][launch row][N]), dense b, at most 3
+// digits. In ksum_k a wave's seven keys each cost it two ChaCha12 rounds (the second for the chunk's one or two rejected
+// words), and the K ciphertexts of a launch repeat them; expanded once, the wave is left with its loads, products and
+// scatter. A key's words are in flight while the one before it is formed. Blocks run ciphertext first, then chunk, then
+// row, each XCD a contiguous range: the ciphertexts share a key's words, and the chunks a row's digits, in one L2.
+template <int NDIG>
+struct SumWords {
+    uint32_t x[NDIG][CS], b[NDIG][CS], a[NDIG][CS], c0[CS];
+};
+template <int NDIG>
+__global__ void __launch_bounds__(CW, NDIG < 3 ? 3 : 2) ksum_pre_k(KsKeyArgs G, const uint32_t* ka, int logn) {
+    __shared__ uint32_t lds[2 * CCH];
+    const KsArgs& A = G.ks;
+    const KeyTab& T = G.key;
+    const int lane = threadIdx.x;
+    const uint32_t l = xcd_block(blockIdx.x, gridDim.x), chunks = (1u << logn) / CCH;
+    const uint32_t c = l % A.K, y = l / A.K / chunks;
+    const uint32_t oc0 = l / A.K % chunks * CCH;
+    const int t = (int)sload(A.rows + y);
+    const bool isq = t < A.nq;
+    Row R = make_row(A.pr[t], logn, lds, 0);
+    const uint32_t p = R.p;
+    const size_t roff = (size_t)t << logn;
+    const int m0 = A.c0_mode & 3;
+    // the c0 term as one more product: times P mod q_t (none on the special rows), or 1
+    const uint32_t f = m0 == 1 ? (isq ? ((const uint32_t*)A.pmod)[t] : 0) : m0 == 2 ? 1 : 0;
+    const int dt = isq ? A.digit_of[t] : -1;
+    const uint32_t* c1 = (const uint32_t*)A.c1 + c * A.ct_stride + roff;
+    const uint32_t* mu = (const uint32_t*)A.modup + c * A.mu_ct_stride + roff;
+    const uint32_t* c0 = m0 ? (const uint32_t*)A.c0 + c * A.ct_stride + roff : c1;
+    const size_t slot = (size_t)slot_of(T, t, A.nq) * T.row_words;
+    auto load = [&](int r, SumWords<NDIG>& w) {
+        const uint32_t kx = sload(A.autok + r) & R.mask2n;
+        const uint32_t s0 = (automorph_slot(inv_odd(kx) & R.mask2n, oc0, logn) & ~(uint32_t)(CCH - 1)) + lane * CS;
+        const gptr kb = as_global(sload(T.kb + r)) + slot + s0;
+        const uint32_t* a = ka + (((size_t)r * NDIG * A.nrows + y) << logn) + s0;
+#pragma unroll
+        for (int d = 0; d < NDIG; ++d) {
+            ld8((d == dt ? c1 : mu + d * A.mu_digit_stride) + s0, w.x[d]);
+            ld8(kb + (uint64_t)d * T.srows * T.row_words, w.b[d]);
+            ld8(a + (((size_t)d * A.nrows) << logn), w.a[d]);
+        }
+        if (f) ld8(c0 + s0, w.c0);
+    };
+    uint32_t acc0[CS], acc1[CS];
+#pragma unroll
+    for (int k = 0; k < CS; ++k) acc0[k] = acc1[k] = 0;
+    auto add = [&](int r, const SumWords<NDIG>& w) {
+        const uint32_t kx = sload(A.autok + r) & R.mask2n;
+        const uint32_t s0 = (automorph_slot(inv_odd(kx) & R.mask2n, oc0, logn) & ~(uint32_t)(CCH - 1)) + lane * CS;
+        uint32_t v0[CS], v1[CS], w0[CS], w1[CS];
+#pragma unroll
+        for (int k = 0; k < CS; ++k) {
+            // at most 4 products of (p - 1)^2 < 2^64
+            uint64_t z0 = f ? (uint64_t)w.c0[k] * f : 0, z1 = 0;
+#pragma unroll
+            for (int d = 0; d < NDIG; ++d) {
+                z0 += (uint64_t)w.x[d][k] * w.b[d][k];
+                z1 += (uint64_t)w.x[d][k] * w.a[d][k];
+            }
+            v0[k] = R.red(z0);
+            v1[k] = R.red(z1);
+        }
+        to_output(R, kx, s0, lane, v0, v1, w0, w1);
+#pragma unroll
+        for (int k = 0; k < CS; ++k) {
+            acc0[k] = addm(acc0[k], w0[k], p);
+            acc1[k] = addm(acc1[k], w1[k], p);
+        }
+    };
+    SumWords<NDIG> wa, wb;
+    load(0, wa);
+    for (int r = 0; r < A.R; r += 2) {
+        if (r + 1 < A.R) load(r + 1, wb);
+        add(r, wa);
+        if (r + 1 >= A.R) break;
+        if (r + 2 < A.R) load(r + 2, wa);
+        add(r + 1, wb);
+    }
+    const size_t o0 = c * A.out_ct_stride + roff + oc0 + lane * CS;
+    uint32_t* out0 = (uint32_t*)A.out0 + o0;
+    uint32_t* out1 = (uint32_t*)A.out1 + o0;
+    if (A.c0_mode & PC_KS_ACC) {
+        uint32_t e0[CS], e1[CS];
+        ld8(out0, e0);
+        ld8(out1, e1);
+#pragma unroll
+        for (int k = 0; k < CS; ++k) {
+            acc0[k] = addm(acc0[k], e0[k], p);
+            acc1[k] = addm(acc1[k], e1[k], p);
+        }
+    }
+    st8(out0, acc0);
+    st8(out1, acc1);
+}
+
 // ------------------------------------------------------------------------------------------------ ks_dot_regen
 // One key (b from key 0 of the KeyTab when key.kb is set, else the dense prime-id rows of ks.kb[0]; `a` regenerated
 // from the args' seed for every digit), K <= 4 ciphertexts, no automorphism, no c0 term; out0 / out1, or through the
@@ -674,6 +771,25 @@ int ks_dot_key_sum(int logn, const KsKeyArgs* g, pc_stream_t s) {
     hipStream_t st = (hipStream_t)s;
     if (a.ndig > 4) hipLaunchKernelGGL(ksum_k<true>, grid, dim3(CW), lds_bytes(nreg), st, *g, logn);
     else hipLaunchKernelGGL(ksum_k<false>, grid, dim3(CW), lds_bytes(nreg), st, *g, logn);
+    return launch_rc();
+}
+
+// ks_dot_key_sum over `a` words expanded by kska_expand; -2 outside its range (dense full-layout keys, 1 to 3 digits)
+int ks_dot_key_sum_pre(int logn, const KsKeyArgs* g, const uint32_t* ka, pc_stream_t s) {
+    using namespace cts;
+    const KsArgs& a = g->ks;
+    if (!ka || a.nrows < 1 || a.R < 1 || a.K < 1) return -1;
+    if (!a.rows || !a.pr || !a.c1 || !a.out0 || !a.out1 || !a.digit_of || !a.autok || !a.modup || !g->key.kb) return -1;
+    if ((a.c0_mode & 3) == 1 && (!a.c0 || !a.pmod)) return -1;
+    if ((a.c0_mode & 3) == 2 && !a.c0) return -1;
+    if ((a.c0_mode & 3) == 3) return -1;
+    if (a.ndig < 1 || a.ndig > 3 || g->key.bits != 0 || (g->key.row_words & 3) || logn < 12 || logn > 16) return -2;
+    if ((a.ct_stride | a.mu_ct_stride | a.mu_digit_stride | a.out_ct_stride) & 3) return -2;
+    const dim3 grid((1u << logn) / CCH * a.nrows * a.K);
+    hipStream_t st = (hipStream_t)s;
+    if (a.ndig == 1) hipLaunchKernelGGL(ksum_pre_k<1>, grid, dim3(CW), 0, st, *g, ka, logn);
+    if (a.ndig == 2) hipLaunchKernelGGL(ksum_pre_k<2>, grid, dim3(CW), 0, st, *g, ka, logn);
+    if (a.ndig == 3) hipLaunchKernelGGL(ksum_pre_k<3>, grid, dim3(CW), 0, st, *g, ka, logn);
     return launch_rc();
 }
 

@@ -322,6 +322,9 @@ struct pcx_rows {
     Dev dev;
 };
 
+// keys whose `a` words a summed rotation expands at a time: a radix-8 rung's seven and one more
+constexpr int ASUM_KEYS = 8;
+
 struct pcx_ctx {
     uint32_t logn = 0, n = 0;
     int nq = 0, kp = 0, dnum = 0, alpha = 0, k_rot = 1, rows = 0;
@@ -353,6 +356,7 @@ struct pcx_ctx {
     std::vector<Level> levels;
     uint32_t *coef = nullptr, *digits = nullptr, *ext = nullptr, *conv = nullptr;
     uint32_t* tmp = nullptr;  // one ciphertext: the rescale's correction rows, a product's d2 (part 1)
+    uint32_t* asum = nullptr; // a summed rotation's expanded `a` words: ASUM_KEYS keys of every digit and row
     size_t ws_bytes = 0;
     // stage timing (pcx_timing): event pairs recorded around each stage's launches on the launch stream
     bool timing = false;
@@ -921,6 +925,13 @@ int modup(pcx_ctx* c, const void* ct, int top, pc_stream_t s, int K = 1) {
     return nt_fwd(c, &f, s);
 }
 
+// Whether a sum of rotations expands its keys' `a` words first (kska_expand) and reads them for every ciphertext: keys
+// with a retry table, full rows, nothing resident. The six ciphertexts of a C4 scoring: a rung's dots 168 us (ksum_k, each
+// ciphertext regenerating the seven keys) -> 54 us
+bool sum_pre(const pcx_ctx* c, const pcx_keys* k, const Level* L) {
+    return k->pval && !c->table_only && k->bits == 0 && k->q_top < 0 && L->ndig <= 3 && !(k->ka && k->regen < L->ndig);
+}
+
 // the dot of keys [r0, r0 + m) of k into m extended ciphertexts at ext (crates/pc-gpu/src/ks.rs:1225-1308 dot_key);
 // sum: 1 sums the m rotations into ext's first ciphertext (KS_SUM), 2 adds that sum onto it (KS_SUM | KS_ACC)
 // K consecutive ciphertexts (ct_words apart, their digits dnum rows N apart) against the same keys: extended
@@ -928,7 +939,9 @@ int modup(pcx_ctx* c, const void* ct, int top, pc_stream_t s, int K = 1) {
 int dot(pcx_ctx* c, pcx_keys* k, int r0, int m, const void* ct, int top, void* ext, pc_stream_t s, int sum = 0,
         int c0_mode = 1, int K = 1, const uint32_t* digits = nullptr, const void* c0 = nullptr) {
     const Level* L = level(c, top);
-    if (!L || r0 < 0 || m < 1 || r0 + m > k->nkeys || K < 1 || K > c->k_max || K > 4) return -1;
+    if (!L || r0 < 0 || m < 1 || r0 + m > k->nkeys || K < 1 || K > c->k_max) return -1;
+    const bool pre = sum && sum_pre(c, k, L);
+    if (K > 4 && !pre) return -1;
     if (k->q_top >= 0 && top > k->q_top) return -1;  // above the keys' band
     KsKeyArgs g;
     memset(&g, 0, sizeof g);
@@ -973,6 +986,23 @@ int dot(pcx_ctx* c, pcx_keys* k, int r0, int m, const void* ct, int top, void* e
         a.key_digit_stride = (uint64_t)c->rows * c->n;
     }
     Stage st(c, 3, s);
+    if (pre) {
+        const size_t per_key = (size_t)c->dnum * c->rows * (c->n / 1024);
+        const int most = ASUM_KEYS * c->dnum * c->rows / (L->ndig * L->nks);
+        for (int j = 0; j < m; j += most) {
+            const int r = std::min(most, m - j);
+            const pch::PatchTab P = {k->pidx + (size_t)(r0 + j) * per_key, k->pval, c->dnum, c->rows};
+            if (int e = pch::kska_expand((int)c->logn, k->seed + r0 + j, c->pr, &P, r, L->ndig, L->ks_rows, L->nks, c->asum, s))
+                return e;
+            KsKeyArgs h = g;
+            h.ks.autok = k->autok + r0 + j;
+            h.ks.R = r;
+            h.key.kb = k->kb + r0 + j;
+            if (j) h.ks.c0_mode |= PC_KS_ACC;
+            if (int e = pch::ks_dot_key_sum_pre((int)c->logn, &h, c->asum, s)) return e;
+        }
+        return 0;
+    }
     if (k->pval && !sum && !c->table_only) {
         // the retry values from the key group's table (no redraw in the dot)
         // the table is indexed by the group's key: the launch's key r is the group's r0 + r
@@ -1380,7 +1410,8 @@ pcx_ctx* pcx_ctx_new_k(uint32_t log_n, const uint64_t* primes, int nq, int kp, i
     c->ext = (uint32_t*)c->dev.alloc((c->ext_rows() + 2 * k_max) * rw);
     c->conv = (uint32_t*)c->dev.alloc(next * 2 * R * rw);
     c->tmp = (uint32_t*)c->dev.alloc((size_t)k_max * 2 * R * rw);
-    c->ws_bytes = (coef_rows + (size_t)k_max * dnum * R + 2 * next * 2 * R + 2 * k_max + (size_t)k_max * 2 * R) * rw;
+    c->asum = (uint32_t*)c->dev.alloc((size_t)ASUM_KEYS * dnum * R * rw);
+    c->ws_bytes = ((size_t)ASUM_KEYS * dnum * R + coef_rows + (size_t)k_max * dnum * R + 2 * next * 2 * R + 2 * k_max + (size_t)k_max * 2 * R) * rw;
     if (c->dev.err) {
         *err = c->dev.err;
         delete c;
@@ -1988,12 +2019,14 @@ static int rotate_sum_k(pcx_ctx* c, pcx_keys* k, const int* idx, int n, const vo
         if (idx[j] < 0 || idx[j] >= k->nkeys || k->galois[idx[j]] == 1) return -1;
     const size_t cw = c->ct_words(), dw = (size_t)c->dnum * c->rows * c->n;
     if (int e = modup(c, ct, top, s, K)) return e;
-    // runs of consecutive keys, each one summed dot over up to 4 of the ciphertexts at a time
+    // runs of consecutive keys, each one summed dot over the ciphertexts (up to 4 at a time where the keys' words are
+    // regenerated)
+    const int most = sum_pre(c, k, level(c, top)) ? K : 4;
     for (int j = 0; j < n;) {
         int m = 1;
         while (j + m < n && idx[j + m] == idx[j] + m) ++m;
-        for (int k0 = 0; k0 < K; k0 += 4) {
-            const int kc = std::min(4, K - k0);
+        for (int k0 = 0; k0 < K; k0 += most) {
+            const int kc = std::min(most, K - k0);
             if (int e = dot(c, k, idx[j], m, (const uint32_t*)ct + k0 * cw, top, c->ext + k0 * cw, s, j == 0 ? 1 : 2, 1,
                             kc, c->digits + k0 * dw))
                 return e;

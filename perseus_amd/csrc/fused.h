@@ -60,6 +60,12 @@ int kska_patch_count(int logn, const uint32_t* const* seeds, const PrimeConst* p
                      uint32_t* counts, pc_stream_t s);
 int kska_patch_fill(int logn, const uint32_t* const* seeds, const PrimeConst* pr, int nkeys, int ndig, int rows,
                     const uint32_t* idx, uint32_t* val, pc_stream_t s);
+// The `a` words of keys 0..nkeys-1 of seeds and P (its tables from the first key on), digits 0..ndig-1, prime ids
+// rows[0..nrows-1], the rejected words from P: out[((r ndig + d) nrows + i) N ..]
+int kska_expand(int logn, const uint32_t* const* seeds, const PrimeConst* pr, const PatchTab* P, int nkeys, int ndig,
+                const uint32_t* rows, int nrows, uint32_t* out, pc_stream_t s);
+// ks_dot_key's summed rotations over `a` words expanded there; -2 outside its range (cts.hip)
+int ks_dot_key_sum_pre(int logn, const KsKeyArgs* g, const uint32_t* ka, pc_stream_t s);
 // the fast dot with the retry values read from P instead of redrawn; -2 where the fast dot does not apply. Beside the
 // table entry's c0 modes it takes c0_mode 3 (no counterpart in the reference, which rejects it): both parts of the
 // ciphertext at c0 (the second ct_stride / 2 words after the first) enter the Q rows as P c0 and P c0', so a

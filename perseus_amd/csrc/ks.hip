@@ -839,6 +839,36 @@ __global__ void __launch_bounds__(DBX) patch_k(const uint32_t* const* seeds, con
     }
 }
 
+// The `a` words of one (1024-slot chunk, row, key x digit) per wave, a block per lane; a lane finds its rejected words'
+// redraws from the wave's prefix of their counts, as the fast dot does
+__global__ void __launch_bounds__(DBX) kska_expand_k(const uint32_t* const* seeds, const PrimeConst* pr, PatchTab P, int ndig,
+                                                     const uint32_t* rows, uint32_t* out, int logn) {
+    const int lane = threadIdx.x, r = blockIdx.z / ndig, d = blockIdx.z % ndig;
+    const uint32_t t = sload(rows + blockIdx.y), chunks = (1u << logn) / DCH;
+    const Expander ex((uint32_t)sload(&pr[t].p));
+    const uint32_t* sp = sload(seeds + r);
+    uint32_t seed[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) seed[i] = sload(sp + i);
+    const uint32_t s0 = blockIdx.x * DCH + lane * DS;
+    uint32_t a[DS];
+    chacha12(seed, s0 >> 4, (uint32_t)d, ex.p, TAG_KSKA, a);
+    uint32_t rej = 0;
+#pragma unroll
+    for (int j = 0; j < DS; ++j) {
+        rej |= (uint32_t)(a[j] >= ex.mp) << j;
+        a[j] = ex.red(a[j]);
+    }
+    if (__ballot(rej != 0)) {
+        uint32_t o = sload(P.idx + (((size_t)r * P.ndig + d) * P.rows + t) * chunks + blockIdx.x) +
+                     lane_prefix(__builtin_popcount(rej), lane);
+#pragma unroll
+        for (int j = 0; j < DS; ++j)
+            if (rej >> j & 1) a[j] = P.val[o++];
+    }
+    st16(out + (((size_t)blockIdx.z * gridDim.y + blockIdx.y) << logn) + s0, a);
+}
+
 // ks_dot: K <= 8 ciphertexts x R keys stored dense (crates/pc-host/src/ks.rs:139-162: KS_SUM -3, K > 8 -1)
 template <int LOGN>
 int ks_dot(const KsArgs* a, pc_stream_t s) {
@@ -1304,6 +1334,14 @@ static int patch_launch(bool fill, int logn, const uint32_t* const* seeds, const
                                  counts, idx, val);
     else hipLaunchKernelGGL(ks::patch_k<false>, grid, dim3(ks::DBX), 0, (hipStream_t)s, seeds, pr, ndig, rows, logn,
                             counts, idx, val);
+    return launch_rc();
+}
+int kska_expand(int logn, const uint32_t* const* seeds, const PrimeConst* pr, const PatchTab* P, int nkeys, int ndig,
+                const uint32_t* rows, int nrows, uint32_t* out, pc_stream_t s) {
+    if (!seeds || !pr || !P || !P->idx || !P->val || !rows || !out) return -1;
+    if (logn < 12 || logn > 16 || nkeys < 1 || ndig < 1 || ndig > P->ndig || nrows < 1) return -1;
+    hipLaunchKernelGGL(ks::kska_expand_k, dim3((1u << logn) / ks::DCH, nrows, nkeys * ndig), dim3(ks::DBX), 0,
+                       (hipStream_t)s, seeds, pr, *P, ndig, rows, out, logn);
     return launch_rc();
 }
 int kska_patch_count(int logn, const uint32_t* const* seeds, const PrimeConst* pr, int nkeys, int ndig, int rows,
