@@ -358,6 +358,241 @@ __global__ void __launch_bounds__(64 * MW, 4) mf_inv_rows(NttArgs A, MfTab T, in
     }
 }
 
+// ------------------------------------------------------------------------------------------------ one pass
+// Rows of at most 2^14 words stay in one workgroup's LDS between the column and the row pass: a launch instead of two, and
+// each word read and written once. The tiles and steps are the two passes'. GEN: as mf_fwd_cols (RsGen).
+//
+// Bound: small launches by their chain of reads and barriers (12 rows of N = 2^12: 5.7 us, the two passes 7.6; of 2^13 7.2
+// and 8.0), large ones by the VALU (1600 rows of N = 2^14: 62 us, the two passes 72). One row of N = 2^14 is eight tiles for
+// each of its CU's waves: 10.6 us where the two passes spread it over several CUs and take 7.8, so it takes this form
+// from ONE14_ROWS rows on.
+constexpr int ONE14_ROWS = 512;
+template <int LOGN>
+struct Mo {
+    using M = Mg<LOGN>;
+    static constexpr int T = M::N / 256;            // tiles
+    static constexpr int MT = LOGN == 14 ? 8 : 4;   // per wave
+    static constexpr int W = T / MT;
+    // Word (r, c) of the row sits at r C + (c with its 16-word block xor g(r)): the four rows that a column step's wave
+    // touches at once (4 apart, R / 16 apart) and the two or four rows of a row tile then sit in distinct blocks
+    static __device__ __forceinline__ uint32_t pos(uint32_t r, uint32_t c) {
+        const uint32_t g = M::C == 128 ? ((r >> 2) & 3) ^ ((r >> 4) & (M::T1 == 8 ? 1 : 3)) ^ ((r & 1) << 1)
+                                       : ((r >> 2) & 3) ^ ((r >> 4) & 3) ^ (r & 3);
+        return r * M::C + (c ^ (g << 4));
+    }
+};
+// Four consecutive words at offset o of a (its row and position in it) through the epilogue
+template <int EPI, int CAN>
+__device__ __forceinline__ void mf_out(const NttArgs& A, size_t o, const uint32_t (&y)[4], uint32_t s, uint32_t ss,
+                                       const MfPrime& P) {
+    uint4 z = make_uint4(mf_canon<CAN>(y[0], P), mf_canon<CAN>(y[1], P), mf_canon<CAN>(y[2], P), mf_canon<CAN>(y[3], P));
+    if (EPI == 0) {
+        *(uint4*)((uint32_t*)A.base + o) = z;
+        return;
+    }
+    const uint32_t* exb = (const uint32_t*)A.ex + o;
+    uint4 ex = ld4(exb);
+    for (int k = 1; k < A.xnum; ++k) {
+        const uint4 e = ld4(exb + k * A.xstride);
+        ex.x = addm(ex.x, e.x, P.p), ex.y = addm(ex.y, e.y, P.p);
+        ex.z = addm(ex.z, e.z, P.p), ex.w = addm(ex.w, e.w, P.p);
+    }
+    uint32_t* eo = (uint32_t*)A.eout + o;
+    uint4 d = make_uint4(0, 0, 0, 0);
+    if (EPI == 2) d = ld4(A.ed ? (const uint32_t*)A.ed + o : eo);
+    auto fin = [&](uint32_t v, uint32_t e, uint32_t dd) {
+        if (EPI == 3) return addm(shoup(e, s, ss, P.p), v, P.p);
+        const uint32_t y1 = shoup(e - v + P.p, s, ss, P.p);
+        return EPI == 2 ? addm(dd, y1, P.p) : y1;
+    };
+    *(uint4*)eo = make_uint4(fin(z.x, ex.x, d.x), fin(z.y, ex.y, d.y), fin(z.z, ex.z, d.z), fin(z.w, ex.w, d.w));
+}
+template <int LOGN, int EPI, int CAN, bool GEN = false>
+__global__ void __launch_bounds__(64 * Mo<LOGN>::W, 4) mf_fwd_one(NttArgs A, MfTab T, RescaleArgs R = {}) {
+    using O = Mo<LOGN>;
+    using M = Mg<LOGN>;
+    constexpr int MT = O::MT;
+    __shared__ uint32_t lds[M::N];
+    const int i = __builtin_amdgcn_readfirstlane(xcd_block(blockIdx.x, gridDim.x));
+    const int pid = __builtin_amdgcn_readfirstlane(row_prime(A, i));
+    const MfLane L;
+    const MfPrime P(A.pr, pid);
+    const size_t row = row_off(A, i) << LOGN;
+    const Buf bs(A.soff ? (const uint32_t*)A.src + ((size_t)A.soff[i] << LOGN) : (const uint32_t*)A.base + row,
+                 (uint32_t)M::N * 4);
+    const uint32_t* tw = T.tw + (size_t)pid * M::TWN;
+    {
+        const uint32_t tau = (uint32_t)(L.w * MT % M::T1), col = (uint32_t)(L.w * MT / M::T1 * 16 + L.j);
+        uint32_t x[MT][4];
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const uint32_t vo = (tau + M::T1 * L.q) * M::C + col, so = (uint32_t)((t + M::T1 * 4 * v) * M::C);
+                if constexpr (GEN) x[t][v] = RsGen(R, (const uint32_t*)A.base + row, pid, LOGN)(vo + so);
+                else x[t][v] = bs.ld(vo * 4, so * 4);
+            }
+        MfMat X, Y;
+        MfInit<true> cx;
+        MfInit<false> cy;
+        X.load(T, pid, MF_X1, L.lane);
+        cx.template load<16>(T, pid, MF_X1, L.lane);
+        Y.load(T, pid, MF_Y1, L.lane);
+        cy.template load<M::T1>(T, pid, MF_Y1, L.lane);
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+            mf_apply(x[t], X, cx, P);
+#pragma unroll
+            for (int m = 0; m < 4; ++m) lds[O::pos(tau + t + M::T1 * (4 * m + L.q), col)] = x[t][m];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+            const uint32_t r = 16 * (tau + t) + 4 * L.q;
+            uint32_t y[4];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) y[v] = lds[O::pos(r + v, col)];
+            mf_twist(y, ld4(tw + M::TW1 + r), P);
+            mf_apply(y, Y, cy, P);
+            // the wave's own words, read by no other before the barrier
+#pragma unroll
+            for (int m = 0; m < 4; ++m) lds[O::pos(r + m, col)] = y[m];
+        }
+    }
+    MfMat X, Y;
+    MfInit<false> cx, cy;
+    X.load(T, pid, MF_X16, L.lane);
+    cx.template load<16>(T, pid, MF_X16, L.lane);
+    Y.load(T, pid, MF_Y2, L.lane);
+    cy.template load<M::S>(T, pid, MF_Y2, L.lane);
+    const uint32_t pos = 16 * L.j + 4 * L.q;
+    const uint4 xi = ld4(tw + M::XI + pos % M::C);
+    uint32_t s = 0, ss = 0;
+    if (EPI) s = sload((const uint32_t*)A.es + pid), ss = sload((const uint32_t*)A.ess + pid);
+    const int bl = L.j / M::S, jj = L.j % M::S;
+    const uint32_t b0 = (uint32_t)(L.w * MT * M::TB);  // the wave's first block
+    __syncthreads();
+    uint32_t x[MT][4];
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) x[t][v] = lds[O::pos(b0 + t * M::TB + bl, (4 * v + L.q) * M::S + jj)];
+    wave_sync();
+    uint32_t* l = lds + L.w * MT * 256;
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+        mf_twist(x[t], ld4(tw + M::TW2 + (b0 + t * M::TB + bl) * 16 + 4 * L.q), P);
+        mf_apply(x[t], X, cx, P);
+#pragma unroll
+        for (int m = 0; m < 4; ++m) l[t * 256 + mf_pos(bl * M::C + (4 * m + L.q) * M::S + jj)] = x[t][m];
+    }
+    wave_sync();
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+        const uint4 y4 = ld4(l + t * 256 + mf_pos(pos));
+        uint32_t y[4] = {y4.x, y4.y, y4.z, y4.w};
+        mf_twist(y, xi, P);
+        mf_twist(y, ld4(tw + M::TWB + (b0 + t * M::TB + pos / M::C) * 16 + 4 * L.q), P);
+        mf_apply(y, Y, cy, P);
+        mf_out<EPI, CAN>(A, row + (L.w * MT + t) * 256 + pos, y, s, ss, P);
+    }
+}
+
+template <int LOGN>
+__global__ void __launch_bounds__(64 * Mo<LOGN>::W, 4) mf_inv_one(NttArgs A, MfTab T) {
+    using O = Mo<LOGN>;
+    using M = Mg<LOGN>;
+    constexpr int MT = O::MT;
+    __shared__ uint32_t lds[M::N];
+    const int i = __builtin_amdgcn_readfirstlane(xcd_block(blockIdx.x, gridDim.x));
+    const int pid = __builtin_amdgcn_readfirstlane(row_prime(A, i));
+    const MfLane L;
+    const MfPrime P(A.pr, pid);
+    const RowSrc src = row_src(A, i, LOGN);
+    const uint32_t* tw = T.itw + (size_t)pid * M::TWN;
+    const uint32_t pos = 16 * L.j + 4 * L.q;
+    const uint32_t b0 = (uint32_t)(L.w * MT * M::TB);
+    const int bl = L.j / M::S, jj = L.j % M::S;
+    {
+        const uint32_t* sp = src.p0 + L.w * MT * 256 + pos;
+        uint4 x[MT];
+#pragma unroll
+        for (int t = 0; t < MT; ++t) x[t] = ld4(sp + t * 256);
+        for (int k = 1; k < src.n; ++k)
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
+                const uint4 e = ld4(sp + k * src.stride + t * 256);
+                x[t].x = addm(x[t].x, e.x, P.p), x[t].y = addm(x[t].y, e.y, P.p);
+                x[t].z = addm(x[t].z, e.z, P.p), x[t].w = addm(x[t].w, e.w, P.p);
+            }
+        MfMat X, Y;
+        MfInit<false> cx, cy;
+        Y.load(T, pid, MF_INV + MF_Y2, L.lane);
+        cy.template load<M::S>(T, pid, MF_INV + MF_Y2, L.lane);
+        X.load(T, pid, MF_INV + MF_X16, L.lane);
+        cx.template load<16>(T, pid, MF_INV + MF_X16, L.lane);
+        const uint4 xi = ld4(tw + M::XI + pos % M::C);
+        uint32_t* l = lds + L.w * MT * 256;
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+            uint32_t y[4] = {x[t].x, x[t].y, x[t].z, x[t].w};
+            mf_apply(y, Y, cy, P);
+            mf_twist(y, xi, P);
+            mf_twist(y, ld4(tw + M::TWB + (b0 + t * M::TB + pos / M::C) * 16 + 4 * L.q), P);
+            *(uint4*)(l + t * 256 + mf_pos(pos)) = make_uint4(y[0], y[1], y[2], y[3]);
+        }
+        wave_sync();
+        uint32_t z[MT][4];
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) z[t][v] = l[t * 256 + mf_pos(bl * M::C + (4 * v + L.q) * M::S + jj)];
+        wave_sync();
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+            mf_apply(z[t], X, cx, P);
+            mf_twist(z[t], ld4(tw + M::TW2 + (b0 + t * M::TB + bl) * 16 + 4 * L.q), P);
+#pragma unroll
+            for (int m = 0; m < 4; ++m) lds[O::pos(b0 + t * M::TB + bl, (4 * m + L.q) * M::S + jj)] = z[t][m];
+        }
+    }
+    MfMat X, Y;
+    MfInit<true> cx;
+    MfInit<false> cy;
+    Y.load(T, pid, MF_INV + MF_Y1, L.lane);
+    cy.template load<M::T1>(T, pid, MF_INV + MF_Y1, L.lane);
+    X.load(T, pid, MF_INV + MF_X1, L.lane);
+    cx.template load<16>(T, pid, MF_INV + MF_X1, L.lane);
+    const uint32_t s = A.es ? sload((const uint32_t*)A.es + i) : sload((const uint32_t*)A.ninv + pid);
+    const uint32_t ss = A.es ? sload((const uint32_t*)A.ess + i) : sload((const uint32_t*)A.ninvs + pid);
+    const uint32_t tau = (uint32_t)(L.w * MT % M::T1), col = (uint32_t)(L.w * MT / M::T1 * 16 + L.j);
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+        const uint32_t r = 16 * (tau + t) + 4 * L.q;
+        uint32_t y[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) y[v] = lds[O::pos(r + v, col)];
+        mf_apply(y, Y, cy, P);
+        mf_twist(y, ld4(tw + M::TW1 + r), P);
+#pragma unroll
+        for (int m = 0; m < 4; ++m) lds[O::pos(r + m, col)] = y[m];
+    }
+    __syncthreads();
+    const Buf bo((const uint32_t*)A.base + (row_off(A, i) << LOGN), (uint32_t)M::N * 4);
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+        uint32_t y[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) y[v] = lds[O::pos(tau + t + M::T1 * (4 * v + L.q), col)];
+        mf_apply(y, X, cx, P);
+#pragma unroll
+        for (int m = 0; m < 4; ++m)
+            bo.st(shoup(y[m], s, ss, P.p), ((tau + M::T1 * L.q) * M::C + col) * 4,
+                  (uint32_t)((t + M::T1 * 4 * m) * M::C) * 4);
+    }
+}
+
 // ------------------------------------------------------------------------------------------------ launchers
 inline int mf_check(const NttArgs* a, const MfTab* t, bool fwd) {
     if (!a || !t || a->nrows < 0 || !a->base || !a->roff || !a->rprime || !a->pr) return -1;
@@ -370,6 +605,23 @@ inline int mf_check(const NttArgs* a, const MfTab* t, bool fwd) {
     }
     if (!fwd && !a->es && (!a->ninv || !a->ninvs)) return -1;
     return 0;
+}
+// whether a whole transform of rows of N takes the one-pass form
+template <int LOGN>
+bool mf_one(int rows) { return rows > 0 && (LOGN <= 13 || rows >= ONE14_ROWS); }
+template <int LOGN, int CAN>
+void mf_one_launch(const NttArgs& A, const MfTab& T, const RescaleArgs* R, hipStream_t st) {
+    const dim3 g(A.nrows), b(64 * Mo<LOGN>::W);
+    if (R) {
+        hipLaunchKernelGGL((mf_fwd_one<LOGN, 3, CAN, true>), g, b, 0, st, A, T, *R);
+        return;
+    }
+    switch (A.epi) {
+        case 0: hipLaunchKernelGGL((mf_fwd_one<LOGN, 0, CAN>), g, b, 0, st, A, T, RescaleArgs{}); break;
+        case 1: hipLaunchKernelGGL((mf_fwd_one<LOGN, 1, CAN>), g, b, 0, st, A, T, RescaleArgs{}); break;
+        case 2: hipLaunchKernelGGL((mf_fwd_one<LOGN, 2, CAN>), g, b, 0, st, A, T, RescaleArgs{}); break;
+        default: hipLaunchKernelGGL((mf_fwd_one<LOGN, 3, CAN>), g, b, 0, st, A, T, RescaleArgs{}); break;
+    }
 }
 template <int LOGN, int CAN>
 void mf_rows_launch(const NttArgs& B, const MfTab& T, int r0, int n, hipStream_t st) {
@@ -388,6 +640,13 @@ int mf_fwd(const NttArgs* a, const MfTab* t, pc_stream_t s, bool cols, const Res
     if (R && a->soff) return -1;
     using M = Mg<LOGN>;
     const NttArgs A = *a;
+    if constexpr (LOGN <= 14) {
+        if (cols && (!R || A.epi == 3) && mf_one<LOGN>(A.nrows)) {
+            if (t->can == 1) mf_one_launch<LOGN, 1>(A, *t, R, (hipStream_t)s);
+            else mf_one_launch<LOGN, 2>(A, *t, R, (hipStream_t)s);
+            return launch_rc();
+        }
+    }
     const int chunk = A.chunk > 0 && cols ? A.chunk : (A.nrows > 0 ? A.nrows : 1);
     hipStream_t st = (hipStream_t)s;
     for (int r0 = 0; r0 < A.nrows; r0 += chunk) {
@@ -407,6 +666,12 @@ int mf_inv(const NttArgs* a, const MfTab* t, pc_stream_t s) {
     if (int rc = mf_check(a, t, false)) return rc;
     using M = Mg<LOGN>;
     const NttArgs A = *a;
+    if constexpr (LOGN <= 14) {
+        if (mf_one<LOGN>(A.nrows)) {
+            hipLaunchKernelGGL((mf_inv_one<LOGN>), dim3(A.nrows), dim3(64 * Mo<LOGN>::W), 0, (hipStream_t)s, A, *t);
+            return launch_rc();
+        }
+    }
     const int chunk = A.chunk > 0 ? A.chunk : (A.nrows > 0 ? A.nrows : 1);
     hipStream_t st = (hipStream_t)s;
     for (int r0 = 0; r0 < A.nrows; r0 += chunk) {

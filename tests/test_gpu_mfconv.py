@@ -64,19 +64,22 @@ def test_conversions_equal_the_tables(stream, monkeypatch, logn, nq, kp, dnum, b
 
             def run(f):
                 got = []
-                for table in (False, True):
+                for table, fused in ((False, 3), (True, 3), (False, 0)):  # the last: bconv, then whole transforms
                     ctx.table_only(table)
+                    ctx.conv_fusion(fused)
                     out.zero()
                     f()
                     stream.sync()
                     got.append(out.download((2, 2, ch.rows, ch.n)))
-                ctx.table_only(False)
+                ctx.conv_fusion(3)
                 return got
 
             say(f"[mfconv] N=2^{logn} {nq}+{kp} primes of {bits} bits, top {top}, {tpw} targets, {fill}: rotations")
-            a, b = run(lambda: ctx.rotate_hoisted(keys, [0, 1], x, top, out, stream))
-            assert (a[:, :, : top + 1] == b[:, :, : top + 1]).all()
+            a, b, c = run(lambda: ctx.rotate_hoisted(keys, [0, 1], x, top, out, stream))
+            for y in (b, c):
+                assert (a[:, :, : top + 1] == y[:, :, : top + 1]).all()
             if top >= 2:
                 say("[mfconv]   two products, rescaled (the exact conversion)")
-                a, b = run(lambda: ctx.mul_relin_rescale(keys, x, x, top, out, stream, K=2))
-                assert (a[:, :, : top - 1] == b[:, :, : top - 1]).all()
+                a, b, c = run(lambda: ctx.mul_relin_rescale(keys, x, x, top, out, stream, K=2))
+                for y in (b, c):
+                    assert (a[:, :, : top - 1] == y[:, :, : top - 1]).all()

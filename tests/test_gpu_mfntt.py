@@ -40,9 +40,18 @@ def chain(logn, bits):
 @pytest.mark.parametrize("logn", [12, 13, 14, 15, 16])
 @pytest.mark.parametrize("bits", [28, 29, 30, 31, "mixed", "small"])
 def test_transforms(stream, logn, bits):
+    transforms(stream, logn, bits)
+
+
+def test_transforms_one_pass(stream):
+    """N = 2^14 in one pass: a launch of more rows than the two passes take (N = 2^12 and 2^13 always do)"""
+    transforms(stream, 14, 31, 517)
+
+
+def transforms(stream, logn, bits, rows=0):
     ch = chain(logn, bits)
     n, nq = ch.n, len(ch.q)
-    rows = nq + 3
+    rows = rows or nq + 3
     say(f"[mfntt] N=2^{logn}, {bits}-bit primes, {rows} rows: forward and inverse against the oracle")
     ctx, oc = pa.Context(ch), twin.Ctx(ch.logn, ch.q, ch.p, ch.dnum)
     rng = np.random.default_rng(logn)
