@@ -310,8 +310,8 @@ def c1_leg(pa, with_cpu, reps=50):
 def cts_leg(pa, ch, ctx, keys, seeds, ct, dev, st, with_cpu, B=8, G=8, npts=63, reps=10):
     """A CtS linear-transform stage at the C3 shape: one ModUp, then res_j = sum_{i < B} rot_i(ct) pt_{B j + i} over
     B = 8 hoisted baby rotations (steps 0..7, keys regenerated in-kernel) and G = 8 giant steps of 63 full diagonals
-    (a radix-32 level of a bootstrap's CoeffToSlot), through pcx_cts_stage: two cts_fused_regen launches of four giant
-    steps each, the rotations never stored."""
+    (a radix-32 level of a bootstrap's CoeffToSlot), through pcx_cts_stage: the babies' dots into the context's workspace,
+    then the plaintext dot over the extended rows (the timed kernel of the roofline)."""
     n, top = ch.n, len(ch.q) - 1
     nr = top + 1 + len(ch.p)
     rng = np.random.default_rng(77)
@@ -334,18 +334,15 @@ def cts_leg(pa, ch, ctx, keys, seeds, ct, dev, st, with_cpu, B=8, G=8, npts=63, 
     ctx.timing(0)
     ms = e0.elapsed_ms(e1) / reps
     tot, cnt = ctx.timing_read()["cts"]
-    launch_ms = tot / cnt / 2  # two kernel launches per stage (giant steps 0-3, 4-7)
-    # algorithmic rows per launch (each operand once): c0 and c1, the ModUp targets, the baby keys' b, the launch's
-    # diagonals and its results; the mean of the two launches (32 and 31 diagonals)
-    ell, E = top + 1, ch.dnum * nr
-    base = 2 * ell + (E - ell) + (B - 1) * E + 2 * 4 * nr
-    rows = base + (min(npts, 4 * B) + max(0, npts - 4 * B)) * nr / 2
+    launch_ms = tot / cnt
+    # the plaintext dot's algorithmic rows (each operand once): the rotations, the diagonals and the results
+    rows = 2 * B * nr + npts * nr + 2 * G * nr
     gbps = rows * 4 * n / (launch_ms * 1e-3) / 1e9
     out = {"workload": f"CtS stage, C3 chain at the top limb: B={B} baby rotations (a regenerated in-kernel), G={G} "
                        f"giant steps, {npts} full diagonals",
            "ms_per_stage": round(ms, 4), "stages_per_s": round(1e3 / ms, 1),
            "baby_key_switches_per_s": round((B - 1) * 1e3 / ms, 1),
-           "kernel": "cts_k<regen>: baby key products, the scatter to output order and the diagonal products",
+           "kernel": "pt_dot_reg_k<8, 0>: the rotations times the diagonals, summed per giant step",
            "kernel_ms_per_launch": round(launch_ms, 4),
            "roofline": {"bound": "hbm", "achieved": round(gbps, 1), "peak": HBM_PEAK_GBPS, "unit": "GB/s",
                         "frac": round(gbps / HBM_PEAK_GBPS, 4), "algorithmic_bytes_per_launch": int(rows * 4 * n)}}

@@ -987,10 +987,11 @@ int pcx_rotate_and_sum_k(pcx_ctx* c, pcx_keys* k, const void* x, int top, int64_
 int pcx_rotate_and_sum_noalloc(pcx_ctx* c, pcx_keys* k, const void* x, int top, int64_t start, int64_t stop,
                                int radix_bits, void* out, pc_stream_t s);
 /* One CtS / StC stage's hoisted baby steps and plaintext products (crates/pc-gpu/src/bts/cts.rs:840-960, LtStage::run
- * steps 1 and 2): ModUp of ct's c1 once, then through the table's cts_fused_regen
+ * steps 1 and 2): ModUp of ct's c1 once, then through the table's cts_fused_regen, or, where the rotations fit the
+ * context's workspace and that is faster, by pcx_cts_stage_hoisted's route (the same words):
  *   res_j = sum_{i < B} rot_i(ct) pt_{B j + i},  j < G,
  * in the extended basis (Q rows 0..top and the special rows), rot_0 = P ct and rot_i (i >= 1) the key switch before
- * ModDown by key r0 + i - 1 of the group, its `a` regenerated in the kernel. pts: a DEVICE array of npts device
+ * ModDown by key r0 + i - 1 of the group, its `a` regenerated. pts: a DEVICE array of npts device
  * pointers to diagonals of top + 1 + kp rows (Q rows 0..top, then the special rows) of ptw words; enc the compact index
  * map (0xFFFFFFFF: full rows; 0x7F000000 | s: o >> s; else o & enc). res: G extended ciphertexts, res_j at
  * res + j ct_words. */

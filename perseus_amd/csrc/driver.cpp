@@ -324,6 +324,8 @@ struct pcx_rows {
 
 // keys whose `a` words a summed rotation expands at a time: a radix-8 rung's seven and one more
 constexpr int ASUM_KEYS = 8;
+// baby steps whose rotations a transform stage keeps in its workspace
+constexpr int STAGE_B = 8;
 
 struct pcx_ctx {
     uint32_t logn = 0, n = 0;
@@ -356,7 +358,9 @@ struct pcx_ctx {
     std::vector<Level> levels;
     uint32_t *coef = nullptr, *digits = nullptr, *ext = nullptr, *conv = nullptr;
     uint32_t* tmp = nullptr;  // one ciphertext: the rescale's correction rows, a product's d2 (part 1)
-    uint32_t* asum = nullptr; // a summed rotation's expanded `a` words: ASUM_KEYS keys of every digit and row
+    // a summed rotation's expanded `a` words (ASUM_KEYS keys of every digit and row), or a transform stage's rotations
+    // (STAGE_B extended ciphertexts)
+    uint32_t* asum = nullptr;
     size_t ws_bytes = 0;
     // stage timing (pcx_timing): event pairs recorded around each stage's launches on the launch stream
     bool timing = false;
@@ -1410,8 +1414,9 @@ pcx_ctx* pcx_ctx_new_k(uint32_t log_n, const uint64_t* primes, int nq, int kp, i
     c->ext = (uint32_t*)c->dev.alloc((c->ext_rows() + 2 * k_max) * rw);
     c->conv = (uint32_t*)c->dev.alloc(next * 2 * R * rw);
     c->tmp = (uint32_t*)c->dev.alloc((size_t)k_max * 2 * R * rw);
-    c->asum = (uint32_t*)c->dev.alloc((size_t)ASUM_KEYS * dnum * R * rw);
-    c->ws_bytes = ((size_t)ASUM_KEYS * dnum * R + coef_rows + (size_t)k_max * dnum * R + 2 * next * 2 * R + 2 * k_max + (size_t)k_max * 2 * R) * rw;
+    const size_t wide_rows = (size_t)std::max(ASUM_KEYS * dnum, STAGE_B * 2) * R;
+    c->asum = (uint32_t*)c->dev.alloc(wide_rows * rw);
+    c->ws_bytes = (wide_rows + coef_rows + (size_t)k_max * dnum * R + 2 * next * 2 * R + 2 * k_max + (size_t)k_max * 2 * R) * rw;
     if (c->dev.err) {
         *err = c->dev.err;
         delete c;
@@ -1857,6 +1862,13 @@ int pcx_cts_stage(pcx_ctx* c, pcx_keys* k, int r0, int B, int G, const void* con
     if (!L || !k || k->c != c || B < 1 || G < 1 || npts < 0 || !pts || !ct || !res) return -1;
     if (!serves(k, top)) return -1;
     if (B > 1 && (r0 < 0 || r0 + B - 1 > k->nkeys)) return -1;
+    // The hoisted route where its rotations fit the workspace and the fast dot takes the keys: a key regenerated once per
+    // stage, its rejected words from the retry table, where the fused kernel regenerates it per four giant steps and redraws.
+    // 8 x 8 steps of C3 623 -> 355 us, 5 x 5 of N = 2^12 85 -> 37. One baby step with its few giant steps in one fused
+    // launch stays there (2 x 3 of N = 2^16 45.7 against 47.3 us, 2 x 2 of N = 2^15 51.9 against 53.1; 2 x 6 53.8 against 45.8)
+    if ((B > 2 || (B == 2 && G > 4)) && B <= STAGE_B && npts > 0 && k->pval && k->bits == 0 && k->q_top < 0 &&
+        !c->table_only && L->ndig <= 3)
+        return pcx_cts_stage_hoisted(c, k, r0, B, G, pts, npts, ptw, enc, ct, top, c->asum, res, s);
     if (B > 1)
         if (int e = modup(c, ct, top, s)) return e;
     CtsRegenArgs ra;
