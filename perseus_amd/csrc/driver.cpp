@@ -2167,9 +2167,9 @@ int pcx_rescale_k(pcx_ctx* c, const void* ct, int top, int ndrop, void* out, int
     const Level::Rescale& Z = c->levels[top].rs[ndrop - 1];
     const int R = c->rows;
     Stage st(c, 9, s);
-    if (ct != out)
-        if (int e = copy_q(c, ct, top, out, s, K)) return e;
+    // out of place without a copy: the tops' INTT and the epilogue read ct (a C3 rescale's 60 rows copied took 6.3 us)
     NttArgs in = ntt_args(c, out, Z.intt, k_rows(c, Z.intt, K));
+    if (ct != out) in.src = ct, in.soff = Z.intt.roff;
     if (int e = nt_inv(c, &in, s)) return e;
     RescaleArgs r;
     memset(&r, 0, sizeof r);
@@ -2193,7 +2193,7 @@ int pcx_rescale_k(pcx_ctx* c, const void* ct, int top, int ndrop, void* out, int
     NttArgs f = ntt_args(c, c->tmp, Z.ntt, k_rows(c, Z.ntt, K));
     f.epi = 3;
     f.eout = out;
-    f.ex = out;
+    f.ex = ct;
     f.xnum = 1;
     f.es = Z.k + 4 * R;
     f.ess = Z.k + 5 * R;
