@@ -319,9 +319,9 @@ struct FastWave {
     uint32_t q[FQCAP];  // rejected words: (digit << 16 | slot), then the redrawn value
     uint32_t qn;
 };
-// KW waves (one key each) share the chunk's D and c0 staged in LDS; a launch with fewer keys than KW runs one-wave
-// workgroups that read D and c0 straight from memory (their LDS holds the wave's buffers only), so the chip keeps
-// enough waves in flight on a single key
+// KW waves (one key each) share the chunk's D and c0 staged in LDS. A launch with fewer keys than KW reads D and c0 straight
+// from memory: in workgroups of a wave per digit (dot_split), or of one wave at one digit or with resident `a` (FastLds1:
+// the wave's buffers only)
 struct FastLds {
     uint32_t D[MAXD][PADW];
     uint32_t c0[PADW];
@@ -739,12 +739,126 @@ __global__ void __launch_bounds__(DBX * NW, 3) dot_fast(KsArgs A, KeyTab T, Patc
     }
 }
 
-// the fast dot's launch: one-wave direct workgroups when the launch has fewer keys than a staged workgroup's waves
+// Fewer keys than a staged workgroup's waves: a workgroup has a wave per digit. dot_fast's one-wave form ran its digits'
+// ChaCha12 blocks, loads and sums in one chain, at one to three waves per SIMD; here wave d regenerates a_d and forms D_d b_d
+// and D_d a_d, the 64-bit products are exchanged through LDS, wave 0 reduces and scatters part 0 and wave 1 part 1. Rejected
+// words: from the retry table (PATCH), else redrawn by their lane.
+//
+// Bound: the lanes' 64-byte accesses (16 consecutive words each) and the chain of table reads, ChaCha12, exchange and
+// scatter. Against the one-wave form, same box: a C1 rotation's packed key (256 chunks) 15.6 -> 11.4 us, one C5 key at 61
+// rows 46.8 -> 42.7, four ciphertexts at 51 rows 139 -> 122; one C3 key (29 us) and two digits at 23 rows (17 us) the same.
+template <int NDIG, bool PATCH, int PK>
+__global__ void __launch_bounds__(DBX * NDIG, 3) dot_split(KsArgs A, KeyTab T, PatchTab P, int logn) {
+    static_assert(NDIG >= 2 && NDIG <= MAXD, "a wave per digit, one per part");
+    __shared__ uint64_t ex[2 * (NDIG - 1)][DS][DBX];
+    __shared__ uint32_t bufs[2][DCH];
+    const int lane = threadIdx.x & (DBX - 1), d = __builtin_amdgcn_readfirstlane(threadIdx.x / DBX);
+    const int t = (int)sload(A.rows + blockIdx.y);
+    const PrimeConst& q = A.pr[t];
+    const Red red(q);
+    const uint32_t p = red.p;
+    const Expander xp(p);
+    const int m0 = A.c0_mode & 3;
+    const int ng = (int)gridDim.z / A.K, c = (int)blockIdx.z / ng, r = P.diag ? c : (int)blockIdx.z % ng;
+    const uint32_t chunk0 = blockIdx.x * DCH, s0 = chunk0 + lane * DS;
+    const size_t trow = (size_t)t << logn;
+    const bool isq = t < A.nq;
+    const uint32_t pm = (m0 == 1 || m0 == 3) && isq ? ((const uint32_t*)A.pmod)[t] : 0;
+    const int slot = slot_of(T, t, A.nq);
+    const gptr kb = as_global(sload(T.kb + r)) + (size_t)slot * T.row_words + (size_t)d * T.srows * T.row_words;
+    const uint32_t kexp = sload(A.autok + r);
+    const uint32_t* D = (isq && A.digit_of[t] == d ? (const uint32_t*)A.c1 + (size_t)c * A.ct_stride
+                                                   : (const uint32_t*)A.modup + (size_t)c * A.mu_ct_stride +
+                                                         (size_t)d * A.mu_digit_stride) + trow;
+    uint32_t x[DS], b[DS], cz[DS], a[DS];
+    ld16(as_global(D + s0), x);
+    if constexpr (PK == 0) ld16(kb + s0, b);
+    else ldpk16<PK>(kb, s0, b);
+    // the wave's part's c0 term: part 0 in modes 1 to 3, part 1 in mode 3 (the second part, ct_stride / 2 further on)
+    const bool add = d == 0 ? m0 == 2 || pm != 0 : d == 1 && m0 == 3 && pm != 0;
+    if (add) ld16(as_global((const uint32_t*)A.c0 + (size_t)c * A.ct_stride + (d ? A.ct_stride / 2 : 0) + trow + s0), cz);
+    uint32_t seed[8];
+    const uint32_t* sp = sload(T.seed + r);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) seed[i] = sload(sp + i);
+    chacha12(seed, s0 >> 4, (uint32_t)d, p, TAG_KSKA, a);
+    uint32_t rej = 0;
+#pragma unroll
+    for (int j = 0; j < DS; ++j) rej |= (uint32_t)(a[j] >= xp.mp) << j;
+    uint32_t o = 0;
+    if constexpr (PATCH)
+        o = sload(P.idx + (((size_t)r * P.ndig + d) * P.rows + slot) * ((1u << logn) / DCH) + blockIdx.x) +
+            lane_prefix(__builtin_popcount(rej), lane);
+#pragma unroll
+    for (int j = 0; j < DS; ++j) a[j] = xp.red(a[j]);
+    while (rej) {
+        const int j = __builtin_ctz(rej);
+        rej &= rej - 1;
+        uint32_t v = 0;
+        if constexpr (PATCH) {
+            v = P.val[o++];
+        } else {
+            for (int tt = 1; tt < KSK_T_MAX; ++tt) {
+                v = chacha12_word(seed, (s0 >> 4) + (uint32_t)tt * ((1u << logn) >> 4), (uint32_t)d, p, TAG_KSKA, j);
+                if (v < xp.mp) break;
+            }
+            v = xp.red(v);
+        }
+#pragma unroll
+        for (int k = 0; k < DS; ++k) a[k] = k == j ? v : a[k];
+    }
+    // the products of the part that another wave sums: wave 0 keeps part 0, wave 1 part 1, the others neither
+    uint64_t z[DS];
+#pragma unroll
+    for (int k = 0; k < DS; ++k) {
+        const uint64_t p0 = (uint64_t)x[k] * b[k], p1 = (uint64_t)x[k] * a[k];
+        if (d == 0) ex[NDIG - 1][k][lane] = p1, z[k] = p0;
+        else if (d == 1) ex[0][k][lane] = p0, z[k] = p1;
+        else ex[1][k][lane] = p0, ex[NDIG][k][lane] = p1;
+    }
+    __syncthreads();
+    if (d > 1) return;
+    // at most NDIG products and the c0 term's: 4 of (p - 1)^2 < 2^64
+    uint32_t* buf = bufs[d];
+    const uint32_t mask2n = (2u << logn) - 1;
+    const int sh = logn - 9;
+    const uint32_t cbh = (((2 * brev_n(s0, logn) + 1) * kexp) & mask2n) >> sh;
+    const uint32_t sth = ((kexp << (logn - 3)) & mask2n) >> sh;
+#pragma unroll
+    for (int k = 0; k < DS; ++k) {
+#pragma unroll
+        for (int w = 0; w < NDIG - 1; ++w) z[k] += ex[d * (NDIG - 1) + w][k][lane];
+        if (add && m0 != 2) z[k] += (uint64_t)cz[k] * pm;
+        uint32_t v = red(z[k]);
+        if (add && m0 == 2) v = addm(v, cz[k], p);
+        buf[scat_addr((cbh + brev4(k) * sth) & (DCH - 1))] = v;
+    }
+    wave_sync();
+    const uint32_t rb = scat_addr(__brev((uint32_t)lane) >> 26);
+    uint32_t* out = (uint32_t*)(d ? A.out1 : A.out0) + (size_t)c * A.out_ct_stride + r * A.out_rot_stride +
+                    trow + (automorph_slot(kexp, chunk0, logn) & ~(uint32_t)(DCH - 1)) + lane * DS;
+    uint32_t v[DS];
+#pragma unroll
+    for (int j = 0; j < DS; ++j) v[j] = buf[rb + 32 * brev4(j)];
+    if (A.c0_mode & PC_KS_ACC) {
+        uint32_t e[DS];
+        ld16(out, e);
+#pragma unroll
+        for (int k = 0; k < DS; ++k) v[k] = addm(v[k], e[k], p);
+    }
+    st16(out, v);
+}
+
+// the fast dot's launch: a wave per digit (one digit, or resident `a`: one-wave workgroups) when the launch has fewer keys
+// than a staged workgroup's waves
 template <int NDIG, bool PATCH, int PK = 0, bool RES = false>
 void dot_fast_launch(dim3 grid, const KsArgs& a, const KeyTab& key, const PatchTab& P, int logn, hipStream_t st) {
     if (P.diag || a.R < KW) {
         grid.z = P.diag ? a.K : a.R * a.K;
-        hipLaunchKernelGGL((dot_fast<NDIG, PATCH, 1, PK, RES>), grid, dim3(DBX), 0, st, a, key, P, logn);
+        if constexpr (NDIG >= 2 && !RES)
+            hipLaunchKernelGGL((dot_split<NDIG, PATCH, PK>), grid, dim3(DBX * NDIG), 0, st, a, key, P, logn);
+        else
+            hipLaunchKernelGGL((dot_fast<NDIG, PATCH, 1, PK, RES>), grid, dim3(DBX), 0, st, a, key, P, logn);
     } else {
         hipLaunchKernelGGL((dot_fast<NDIG, PATCH, KW, PK, RES>), grid, dim3(KBX), 0, st, a, key, P, logn);
     }
@@ -805,7 +919,7 @@ int dot_patched(const KsKeyArgs* g, const PatchTab* P, pc_stream_t s) {
     if (!a.rows || !a.pr || !a.c1 || !a.out0 || !a.out1 || !a.autok || !a.digit_of || !a.modup) return -1;
     if ((a.c0_mode & 3) != 0 && (a.c0_mode & 3) != 2 && (!a.c0 || !a.pmod || !a.pmods)) return -1;
     if ((a.c0_mode & 3) == 2 && !a.c0) return -1;
-    if ((a.c0_mode & 3) == 3 && ((a.ct_stride & 1) || a.R >= KW)) return -2;  // mode 3: the one-wave form only
+    if ((a.c0_mode & 3) == 3 && ((a.ct_stride & 1) || a.R >= KW)) return -2;  // mode 3: the forms of few keys only
     if (!key.kb || !key.seed) return -1;
     const int chunks = (1 << LOGN) / DCH;
     int groups = 1;
