@@ -868,8 +868,8 @@ int pcx_ctx_table_only(pcx_ctx* c, int on);
 /* No counterpart in the reference: a tuning switch. Which conversions the driver streams into the forward NTT's
  * column pass instead of the table's bconv then ntt_fwd: bit 0 the ModUp, bit 1 the ModDown the register-held fused
  * form does not take (more than 6 special primes), bit 2 the ModDown-rescale (default 3, or PCX_CC_FUSED at context
- * creation; the table-only mode uses none). mask < 0 reads the setting. Returns the previous mask, -1 on NULL. The
- * words are the same either way. */
+ * creation; the table-only mode uses none). On the matrix cores the ModDown-rescale is streamed under any mask but 0.
+ * mask < 0 reads the setting. Returns the previous mask, -1 on NULL. The words are the same either way. */
 int pcx_ctx_conv_fusion(pcx_ctx* c, int mask);
 
 /* No counterpart in the reference: a tuning switch. Launches of N = 2^16 with at least `rows` rows take the one-pass

@@ -344,8 +344,9 @@ struct pcx_ctx {
     int md_fused_init = 1;    // md_fused as chosen at creation (PCX_MD_FUSED included), restored by table_only(0)
     int table_only = 0;       // every launch through the kernel table (pcx_ctx_table_only)
     // conversions streamed into the NTT column pass (pch::conv_cols), by call site: CC_MODUP | CC_MODDOWN | CC_MDR
-    // (ModDown the fused md_conv_cols does not take, the ModDown-rescale); pcx_ctx_conv_fusion, PCX_CC_FUSED. The
-    // default leaves the ModDown-rescale on bconv then ntt_fwd: its exact form carries the doubles of u beside the sums
+    // (ModDown the fused md_conv_cols does not take, the ModDown-rescale); pcx_ctx_conv_fusion, PCX_CC_FUSED. On the
+    // matrix cores (mfc_on) any nonzero mask streams the ModDown-rescale. The butterflies' form
+    // leaves the ModDown-rescale on bconv then ntt_fwd by default: its exact form carries the doubles of u beside the sums
     // (2 waves per SIMD) and measured slower on the C5 bootstrap (ModUp + ModDown stages 5.09 ms unfused, 4.91 with
     // ModUp and ModDown streamed, 5.22 with the rescale's too; same box)
     int cc_fused = 3;
