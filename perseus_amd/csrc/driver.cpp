@@ -741,14 +741,28 @@ NttArgs ntt_args(const pcx_ctx* c, void* base, const Rows& r, int nrows) {
 }
 
 // The transforms: on the matrix cores (mf.h), or through the kernel table's butterflies where a caller asks for the
-// table alone, for the one-pass form, or where the context's primes are below the matrix passes' range
+// table alone, for the one-pass form, where the context's primes are below the matrix passes' range, or where they are faster
 bool mf_on(const pcx_ctx* c) { return c->mf.can > 0 && !c->table_only; }
+// Where the butterflies stay the faster whole transform (medians of alternating runs on one box, butterflies / matrix):
+//  N = 2^15 past the last-level cache's 256 MB: primes below 2^30 from 2048 rows on (forward 2048 rows 192.7 / 197.3 us,
+//   2560 273 / 302, 4096 449 / 476, inverse 2560 278 / 288; at 1792 rows 161 / 153), 31-bit ones forward above 2112 (2112
+//   rows +1.5% for the matrix form, 2176 -6%, 2560 280 / 304); N = 2^16 gains at every size (2560 rows 576 / 567).
+//  The inverse of few rows of primes below 2^30, whose lazy butterflies are the shorter chain: N = 2^14 12 rows 7.98 / 8.36,
+//   40 rows -2%, 48 even; 2^15 12 rows 8.59 / 8.88, 160 rows -3%, 200 +2%; 2^16 12 rows 9.06 / 9.31, 24 even. At N = 2^12
+//   and 2^13 the one launch always pays (one row 6.5 / 5.2 and 7.3 / 6.7).
+bool mf_ntt_pays(const pcx_ctx* c, int rows, bool fwd) {
+    if (c->logn == 15 && (c->lazy ? rows >= 2048 : fwd && rows > 2112)) return false;
+    return fwd || !c->lazy || c->logn < 14 || rows > (c->logn == 14 ? 40 : c->logn == 15 ? 160 : 16);
+}
+bool mf_ntt_on(const pcx_ctx* c, int rows, bool fwd) {
+    return mf_on(c) && !pch::ntt_one_pass((int)c->logn, rows) && mf_ntt_pays(c, rows, fwd);
+}
 int nt_fwd(const pcx_ctx* c, const NttArgs* a, pc_stream_t s) {
-    if (!mf_on(c) || pch::ntt_one_pass((int)c->logn, a->nrows)) return c->tab->ntt_fwd(a, s);
+    if (!mf_ntt_on(c, a->nrows, true)) return c->tab->ntt_fwd(a, s);
     return pch::mf_ntt_fwd((int)c->logn, a, &c->mf, s);
 }
 int nt_inv(const pcx_ctx* c, const NttArgs* a, pc_stream_t s) {
-    if (!mf_on(c) || pch::ntt_one_pass((int)c->logn, a->nrows)) return c->tab->ntt_inv(a, s);
+    if (!mf_ntt_on(c, a->nrows, false)) return c->tab->ntt_inv(a, s);
     return pch::mf_ntt_inv((int)c->logn, a, &c->mf, s);
 }
 int nt_fwd_rows(const pcx_ctx* c, const NttArgs* a, pc_stream_t s) {

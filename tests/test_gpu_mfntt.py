@@ -43,6 +43,16 @@ def test_transforms(stream, logn, bits):
     transforms(stream, logn, bits)
 
 
+# both sides of the rows from which, or up to which, the butterflies are taken (driver.cpp mf_ntt_pays): the inverse of few
+# rows of primes below 2^30, N = 2^15 past the last-level cache
+@pytest.mark.parametrize("logn,bits,rows", [
+    (14, 28, 40), (14, 30, 41), (15, 28, 160), (15, 30, 161), (16, 28, 16), (16, 30, 17),
+    (15, 30, 2047), (15, 28, 2048), (15, 31, 2112), (15, 31, 2113),
+])
+def test_transforms_at_the_rule(stream, logn, bits, rows):
+    transforms(stream, logn, bits, rows)
+
+
 def test_transforms_one_pass(stream):
     """N = 2^14 in one pass: a launch of more rows than the two passes take (N = 2^12 and 2^13 always do)"""
     transforms(stream, 14, 31, 517)
@@ -52,6 +62,7 @@ def transforms(stream, logn, bits, rows=0):
     ch = chain(logn, bits)
     n, nq = ch.n, len(ch.q)
     rows = rows or nq + 3
+    twin.set_threads(16)
     say(f"[mfntt] N=2^{logn}, {bits}-bit primes, {rows} rows: forward and inverse against the oracle")
     ctx, oc = pa.Context(ch), twin.Ctx(ch.logn, ch.q, ch.p, ch.dnum)
     rng = np.random.default_rng(logn)
