@@ -742,7 +742,9 @@ __global__ void __launch_bounds__(DBX * NW, 3) dot_fast(KsArgs A, KeyTab T, Patc
 // Fewer keys than a staged workgroup's waves: a workgroup has a wave per digit. dot_fast's one-wave form ran its digits'
 // ChaCha12 blocks, loads and sums in one chain, at one to three waves per SIMD; here wave d regenerates a_d and forms D_d b_d
 // and D_d a_d, the 64-bit products are exchanged through LDS, wave 0 reduces and scatters part 0 and wave 1 part 1. Rejected
-// words: from the retry table (PATCH), else redrawn by their lane.
+// words: from the retry table (PATCH), else redrawn by the wave, 64 at a time: each by its own lane, launches that fill the
+// chip lost to the one wave (three rotations by packed keys at 54 rows of N = 2^16: one wave 315 us, lanes 363, wave 310;
+// at 35 rows of a chain that rejects a third of its words 737, 898 and 700).
 //
 // Bound: the lanes' 64-byte accesses (16 consecutive words each) and the chain of table reads, ChaCha12, exchange and
 // scatter. Against the one-wave form, same box: a C1 rotation's packed key (256 chunks) 15.6 -> 11.4 us, one C5 key at 61
@@ -786,27 +788,46 @@ __global__ void __launch_bounds__(DBX * NDIG, 3) dot_split(KsArgs A, KeyTab T, P
 #pragma unroll
     for (int j = 0; j < DS; ++j) rej |= (uint32_t)(a[j] >= xp.mp) << j;
     uint32_t o = 0;
-    if constexpr (PATCH)
+    [[maybe_unused]] uint64_t* rq = ex[d == 0 ? NDIG - 1 : d - 1][0];
+    if constexpr (PATCH) {
         o = sload(P.idx + (((size_t)r * P.ndig + d) * P.rows + slot) * ((1u << logn) / DCH) + blockIdx.x) +
             lane_prefix(__builtin_popcount(rej), lane);
+    } else if (__ballot(rej != 0)) {
+        // the wave's rejected words, a lane each and round, queued in the exchange slab that the wave fills after
+        const uint32_t cnt = __builtin_popcount(rej);
+        o = lane_prefix(cnt, lane);
+        const uint32_t nq = __shfl(o + cnt, DBX - 1);
+        uint32_t m = rej, i = o;
+        while (m) {
+            const int j = __builtin_ctz(m);
+            m &= m - 1;
+            rq[i++] = lane * DS + j;
+        }
+        wave_sync();
+        for (uint32_t e = lane; e < nq; e += DBX) {
+            const uint32_t sl = (uint32_t)rq[e];
+            uint32_t v = 0;
+            for (int tt = 1; tt < KSK_T_MAX; ++tt) {
+                v = chacha12_word(seed, ((chunk0 + sl) >> 4) + (uint32_t)tt * ((1u << logn) >> 4), (uint32_t)d, p, TAG_KSKA,
+                                  (int)(sl & 15));
+                if (v < xp.mp) break;
+            }
+            rq[e] = xp.red(v);
+        }
+        wave_sync();
+    }
 #pragma unroll
     for (int j = 0; j < DS; ++j) a[j] = xp.red(a[j]);
     while (rej) {
         const int j = __builtin_ctz(rej);
         rej &= rej - 1;
-        uint32_t v = 0;
-        if constexpr (PATCH) {
-            v = P.val[o++];
-        } else {
-            for (int tt = 1; tt < KSK_T_MAX; ++tt) {
-                v = chacha12_word(seed, (s0 >> 4) + (uint32_t)tt * ((1u << logn) >> 4), (uint32_t)d, p, TAG_KSKA, j);
-                if (v < xp.mp) break;
-            }
-            v = xp.red(v);
-        }
+        uint32_t v;
+        if constexpr (PATCH) v = P.val[o++];
+        else v = (uint32_t)rq[o++];
 #pragma unroll
         for (int k = 0; k < DS; ++k) a[k] = k == j ? v : a[k];
     }
+    if constexpr (!PATCH) wave_sync();
     // the products of the part that another wave sums: wave 0 keeps part 0, wave 1 part 1, the others neither
     uint64_t z[DS];
 #pragma unroll
@@ -849,16 +870,25 @@ __global__ void __launch_bounds__(DBX * NDIG, 3) dot_split(KsArgs A, KeyTab T, P
     st16(out, v);
 }
 
-// the fast dot's launch: a wave per digit (one digit, or resident `a`: one-wave workgroups) when the launch has fewer keys
-// than a staged workgroup's waves
+// The fast dot's launch: a wave per digit (one digit, or resident `a`: one-wave workgroups) when the launch has fewer keys
+// than a staged workgroup's waves. Without a retry table a wave per digit pays a ChaCha12 round for each digit's few
+// rejected words where the one wave pays one for all. That shows once the SIMDs have more than a workgroup each
+// (SPLIT_REDRAW) at N <= 2^14 or with more than two keys or ciphertexts: 30-bit packed keys, one wave / wave per digit, N = 2^14: 288
+// workgroups 54.5 / 51.0 us, 1120 79.2 / 76.3, 1728 90.6 / 92.9; N = 2^16: one key, 2240 workgroups, 123.4 / 117.5, two,
+// 4480, 167.2 / 159.4, four ciphertexts, 3072, 135.0 / 138.2.
+constexpr long SPLIT_REDRAW = 1200;
+inline bool split_pays(const dim3& g) {
+    return (long)g.x * g.y * g.z <= SPLIT_REDRAW || (g.x > (1 << 14) / DCH && g.z <= 2);
+}
 template <int NDIG, bool PATCH, int PK = 0, bool RES = false>
 void dot_fast_launch(dim3 grid, const KsArgs& a, const KeyTab& key, const PatchTab& P, int logn, hipStream_t st) {
     if (P.diag || a.R < KW) {
         grid.z = P.diag ? a.K : a.R * a.K;
-        if constexpr (NDIG >= 2 && !RES)
-            hipLaunchKernelGGL((dot_split<NDIG, PATCH, PK>), grid, dim3(DBX * NDIG), 0, st, a, key, P, logn);
-        else
+        if (NDIG < 2 || RES || (!PATCH && !split_pays(grid))) {
             hipLaunchKernelGGL((dot_fast<NDIG, PATCH, 1, PK, RES>), grid, dim3(DBX), 0, st, a, key, P, logn);
+        } else if constexpr (NDIG >= 2 && !RES) {
+            hipLaunchKernelGGL((dot_split<NDIG, PATCH, PK>), grid, dim3(DBX * NDIG), 0, st, a, key, P, logn);
+        }
     } else {
         hipLaunchKernelGGL((dot_fast<NDIG, PATCH, KW, PK, RES>), grid, dim3(KBX), 0, st, a, key, P, logn);
     }
