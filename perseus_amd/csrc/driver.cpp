@@ -821,14 +821,30 @@ int mfc_shape(const pcx_ctx* c, const BconvArgs& b) {
     if (c->cc_tpw > 0) return c->cc_tpw > 2 ? (c->cc_tpw + 3) / 4 * 4 : c->cc_tpw;
     return mfc_wgs(c, b, 8) >= 3000 ? 8 : mfc_wgs(c, b, 4) >= 160 ? 4 : 2;
 }
-// Above 8 sources the matrix-core form always pays (46 + 16 primes of N = 2^13, its smallest launches 384 waves: a
-// bootstrap 3098 -> 2746 us). Up to 4 the butterflies' forms sum in registers as fast (2 sources, 12 jobs of N = 2^16: a C4
-// scoring 488 against 491 us; 3 sources, 46 jobs of N = 2^12: 23 rotations 68.6 against 73.1 us). Between, it wants
-// waves to hide its chained reads and barriers: C3's ModDown of one rotation gains by it, five products of N = 2^13 (320
-// waves: 107.1 against 107.8 us) do not.
-bool mfc_on(const pcx_ctx* c, const Bconv& p, const BconvArgs& b) {
+// Whether conversion b of plan p runs on the matrix cores: by sources, N and waves, from each call site timed both ways
+// (5 to 16 sources, N = 2^12 to 2^16, 1 to 26 keys or products, one box; us by which the matrix form is the shorter):
+//  Up to 4 sources the butterflies' forms sum in registers as fast.
+//  N <= 2^13: above 8 sources until the launch fills the chip (9 sources of 2^13: 80 waves +10, 800 +4, 1280 +1.6, 1600 -1,
+//   3200 -7; 16 sources: 2560 +3, 3840 -3), 7 and 8 up to 256 waves (256 +1, 320 -2, 1280 -3), 5 and 6 never (64 -1, 1280 -5).
+//   Exact conversions (bconv's extra pass on the other side): up to 256 waves (+2), above 10 sources 512 (+1, 1280 -2).
+//  N = 2^14: above 8 sources (+4 to +17); 7 and 8 up to 512 waves (+1) and from 1920 on (+2; 640 to 1280 -1 to -2); 5 and 6
+//   from 2560 on (+1; 768 -3). N = 2^15: above 6 sources (+1 to +16), 5 and 6 from 1920 on (+1; 768 -3). Exact: always
+//   (+1 to +10), but for 16 sources or more below 2048 waves (1024 -4: the form of 20 sources spills).
+//  N = 2^16: always above 6 sources (+1 to +22), 5 and 6 from 800 waves on (+2 to +17; 512 -2); exact always (+1 to +25).
+bool mfc_pays(int logn, int src, long waves, bool exact) {
+    if (src <= 4) return false;
+    if (logn <= 13) {
+        if (exact) return waves <= (src > 10 ? 512 : 256);
+        return src > 8 ? waves <= 170 * (src - 1) : src > 6 && waves <= 256;
+    }
+    if (exact) return logn == 16 || src < 16 || waves >= 2048;
+    if (logn == 16) return src > 6 || waves >= 800;
+    if (logn == 15) return src > 6 || waves >= 1920;
+    return src > 8 || (src > 6 ? waves <= 512 || waves >= 1920 : waves >= 2560);
+}
+bool mfc_on(const pcx_ctx* c, const Bconv& p, const BconvArgs& b, bool exact = false) {
     if (!mf_on(c) || p.mf_ns == 0) return false;
-    return c->cc_tpw > 0 || p.mf_src > 8 || (p.mf_src > 4 && mfc_wgs(c, b, 4) << (c->logn / 2) >> 5 >= 800);
+    return c->cc_tpw > 0 || mfc_pays((int)c->logn, p.mf_src, mfc_wgs(c, b, 4) << (c->logn / 2) >> 5, exact);
 }
 // The conversion b of plan p (its first b.njobs jobs) on the matrix cores, fused into the column pass of f's rows, then f's
 // row pass and epilogue. exact: p's jobs are, b.src is the context's extended workspace
@@ -901,7 +917,7 @@ int moddown_rescale(pcx_ctx* c, void* ext, int top, void* out, const void* onto,
     f.xstride = c->ct_words();
     f.es = M.ntt.es;
     f.ess = M.ntt.es + c->rows;
-    if (mfc_on(c, M.conv, b) && c->cc_fused) return mfc_then_rows(c, M.conv, b, f, s, true);
+    if (mfc_on(c, M.conv, b, true) && c->cc_fused) return mfc_then_rows(c, M.conv, b, f, s, true);
     if (cc_on(c, CC_MDR)) return conv_then_rows(c, b, f, s, 5, 6, c->kp + 2, 1);
     {
         Stage st(c, 5, s);

@@ -1,7 +1,7 @@
 """The conversions on the matrix cores (mfconv.hip) against the same context's launches through the kernel table alone
 (bconv, then the transforms), word for word: one to 17 sources (padded to 8, 16 and 20, one more in the exact
-conversion), targets that leave a last run of one to four, every number of targets per workgroup that its rule chooses
-(1, 2, 4, 8: PCX_CC_TPW), every ring degree, 28- to 31-bit primes, and ciphertexts of words at the ends of their range
+conversion), targets that leave a last run of one to four, every number of targets per workgroup (1, 2, 4, 8: PCX_CC_TPW
+forces the form; 0: the context's own choice of form and number), every ring degree, 28- to 31-bit primes, and ciphertexts of words at the ends of their range
 (0, p - 1), where a digit sum that overflowed would show. Each test prints its case before the GPU runs."""
 import sys
 
@@ -40,7 +40,7 @@ CASES = [
 
 
 @pytest.mark.parametrize("logn,nq,kp,dnum,bits,tops", CASES)
-@pytest.mark.parametrize("tpw", [1, 2, 4, 8])
+@pytest.mark.parametrize("tpw", [0, 1, 2, 4, 8])
 def test_conversions_equal_the_tables(stream, monkeypatch, logn, nq, kp, dnum, bits, tops, tpw):
     monkeypatch.setenv("PCX_CC_TPW", str(tpw))
     ch = make("mfc", logn, nq, kp, dnum, bits)
