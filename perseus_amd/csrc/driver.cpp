@@ -1887,6 +1887,18 @@ int pcx_moddown_k(pcx_ctx* c, void* ext, int top, void* out, int m, pc_stream_t 
     return moddown(c, ext, c->conv, m, top, out, s);
 }
 
+// Where one fused launch is the faster stage (every shape of 2 to 8 baby and 1 to 8 giant steps timed both ways at N = 2^12 to
+// 2^16 and 5 to 44 rows): no or one baby rotation and at most four giant steps (2 x 3 of N = 2^16, 6 rows, 36 us against 41;
+// 2 x 5 53 against 44), and one giant step of few baby steps whose waves, one per 512 words of a row, are one round of the
+// chip's 1024 SIMDs but fill it (fused / hoisted, N = 2^15, two digits: 640 waves 3 x 1 -5%, 5 x 1 -3%; 1024 waves 5 x 1
+// -12%, 5 x 2 -5%, 6 x 1 +2%; 1088 waves +5% and more; 512 waves even; 4 and 7 baby steps gain throughout)
+static bool stage_fused(int B, int G, int ndig, long waves) {
+    if (B <= 2) return B == 1 || G <= 4;
+    if (waves < 560 || waves > 1024 || G > (B == 5 && waves > 800 ? 2 : 1)) return false;
+    if (ndig > 2 && (waves <= 800 || B == 3)) return false;
+    return B == 3 || B == 5 || (B == 6 && waves <= 1000);
+}
+
 int pcx_cts_stage(pcx_ctx* c, pcx_keys* k, int r0, int B, int G, const void* const* pts, int npts, int ptw,
                   uint32_t enc, const void* ct, int top, void* res, pc_stream_t s) {
     const Level* L = c ? level(c, top) : nullptr;
@@ -1895,10 +1907,9 @@ int pcx_cts_stage(pcx_ctx* c, pcx_keys* k, int r0, int B, int G, const void* con
     if (B > 1 && (r0 < 0 || r0 + B - 1 > k->nkeys)) return -1;
     // The hoisted route where its rotations fit the workspace and the fast dot takes the keys: a key regenerated once per
     // stage, its rejected words from the retry table, where the fused kernel regenerates it per four giant steps and redraws.
-    // 8 x 8 steps of C3 623 -> 355 us, 5 x 5 of N = 2^12 85 -> 37. One baby step with its few giant steps in one fused
-    // launch stays there (2 x 3 of N = 2^16 45.7 against 47.3 us, 2 x 2 of N = 2^15 51.9 against 53.1; 2 x 6 53.8 against 45.8)
-    if ((B > 2 || (B == 2 && G > 4)) && B <= STAGE_B && npts > 0 && k->pval && k->bits == 0 && k->q_top < 0 &&
-        !c->table_only && L->ndig <= 3)
+    // 8 x 8 steps of C3 623 -> 355 us, 5 x 5 of N = 2^12 85 -> 37
+    if (B <= STAGE_B && npts > 0 && k->pval && k->bits == 0 && k->q_top < 0 && !c->table_only && L->ndig <= 3 &&
+        !stage_fused(B, G, L->ndig, (long)(c->n / 512) * L->nks))
         return pcx_cts_stage_hoisted(c, k, r0, B, G, pts, npts, ptw, enc, ct, top, c->asum, res, s);
     if (B > 1)
         if (int e = modup(c, ct, top, s)) return e;

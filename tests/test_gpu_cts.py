@@ -1,6 +1,6 @@
 """Parity of the fused CtS stage (hoisted baby rotations times the BSGS diagonals) with the oracle, word for word:
-the driver's stage (ModUp + cts_fused_regen) and the kernel table's two entries called directly with the ABI structs
-(crates/pc-kernels/kernels/cts.cuh; args.cuh CtsArgs / CtsRegenArgs). Each test prints its case before the GPU runs.
+the driver's stage (ModUp, then cts_fused_regen or the hoisted rotations) and the kernel table's two entries called
+directly with the ABI structs (crates/pc-kernels/kernels/cts.cuh; args.cuh CtsArgs / CtsRegenArgs). Each test prints its case before the GPU runs.
 """
 import ctypes as C
 import sys
@@ -11,6 +11,8 @@ import pytest
 import perseus_amd as pa
 from perseus_amd import abi
 from perseus_amd._lib import LIB
+from perseus_amd.chains import make
+from perseus_amd.engine import band_rows
 from tests import twin
 
 pytestmark = pytest.mark.gpu
@@ -34,8 +36,8 @@ _CTX = {}
 
 def contexts(name):
     if name not in _CTX:
-        ch = pa.preset(name)
-        _CTX[name] = (ch, pa.Context(ch, k_rot=4), twin.Ctx(ch.logn, ch.q, ch.p, ch.dnum))
+        ch = pa.preset(name) if isinstance(name, str) else make("cts", *name)
+        _CTX[name] = (ch, pa.Context(ch, k_rot=5), twin.Ctx(ch.logn, ch.q, ch.p, ch.dnum))
     return _CTX[name]
 
 
@@ -85,12 +87,21 @@ def oracle_keys(oc, ch, steps, seed):
     ("c3", 5, 2, 10, FULL, 29, 0),            # the C3 chain at its full shape
     ("rej", 4, 2, 8, FULL, 5, 0),             # a third of the KSKA words rejected: the wave's redraw queue
     ("small28", 9, 4, 33, FULL, 5, 28),       # 28-bit primes, more than 8 baby steps: the reference's own regime
+    # the lines of pcx_cts_stage's own choice: two baby steps at 4 and 5 giant steps, 8 and 9 baby steps, and 640 and 512
+    # waves of 5 x 1 steps
+    ("rej", 2, 4, 8, FULL, 5, 0),
+    ("small", 2, 5, 9, FULL, 5, 0),
+    ("small", 8, 2, 16, 0x7F000003, 4, 0),
+    ("rej", 9, 2, 17, FULL, 5, 0),
+    ((14, 15, 5, 2, 30), 5, 1, 5, FULL, 14, 0),
+    ((14, 12, 4, 2, 30), 5, 1, 5, FULL, 11, 0),
 ])
-@pytest.mark.parametrize("route", ["fused", "hoisted"])
+@pytest.mark.parametrize("route", ["fused", "stage", "hoisted"])
 def test_cts_stage(stream, name, B, G, npts, enc, top, bits, route):
-    """pcx_cts_stage (fused: the cts_fused_regen kernel) and pcx_cts_stage_hoisted (P ct, the babies' dots into a
-    workspace of extended ciphertexts, pt_dot over the extended rows) against the oracle's fused stage; the hoisted
-    route's results then through pcx_moddown_k (all G in one launch sequence) against the oracle's ModDown of each."""
+    """pcx_cts_stage through the kernel table (fused: cts_fused_regen), by its own choice of route (stage), and
+    pcx_cts_stage_hoisted (P ct, the babies' dots into a workspace of extended ciphertexts, pt_dot over the extended rows)
+    against the oracle's fused stage; the hoisted route's results then through pcx_moddown_k (all G in one launch sequence)
+    against the oracle's ModDown of each."""
     say(f"[cts stage] {route} {name} B={B} G={G} npts={npts} enc={enc:#x} top={top} bits={bits}")
     ch, ctx, oc = contexts(name)
     twin.set_threads(16)
@@ -105,8 +116,12 @@ def test_cts_stage(stream, name, B, G, npts, enc, top, bits, route):
     ptrs = dev_ptrs(pbufs)
     dev = pa.DevBuf.from_array(ct)
     res = ctx.ct_buf(G)
-    if route == "fused":
-        ctx.cts_stage(keys, 0, B, G, ptrs, npts, ptw, enc, dev, top, res, stream)
+    if route != "hoisted":
+        prev = ctx.table_only(route == "fused")
+        try:
+            ctx.cts_stage(keys, 0, B, G, ptrs, npts, ptw, enc, dev, top, res, stream)
+        finally:
+            ctx.table_only(prev)
     else:
         rot = ctx.ct_buf(B)
         ctx.cts_stage_hoisted(keys, 0, B, G, ptrs, npts, ptw, enc, dev, top, rot, res, stream)
@@ -125,6 +140,28 @@ def test_cts_stage(stream, name, B, G, npts, enc, top, bits, route):
         for j in range(G):
             wq = oc.moddown(want[j].copy(), top)
             assert (gq[j][:, : top + 1] == wq[:, : top + 1]).all(), f"moddown {j}"
+
+
+def test_cts_stage_banded(stream):
+    """a stage of banded keys (b rows up to the band's top): the fused kernel, four baby steps"""
+    say("[cts stage] small, keys banded at 4, top 3")
+    ch, ctx, oc = contexts("small")
+    rng = np.random.default_rng(53)
+    B, G, npts, top, q_top = 4, 2, 8, 3, 4
+    gals, seeds, bs = oracle_keys(oc, ch, [1, 2, 7], seed=19)
+    keys = pa.Keys(ctx, gals, seeds=seeds, b=[band_rows(b, ctx, q_top) for b in bs], bits=0, q_top=q_top)
+    ct = random_ct(ch, top, rng)
+    pts = diagonals(ch, top, npts, ch.n, rng)
+    pbufs = [pa.DevBuf.from_array(p) for p in pts]
+    ptrs, dev, res = dev_ptrs(pbufs), pa.DevBuf.from_array(ct), ctx.ct_buf(G)
+    ctx.cts_stage(keys, 0, B, G, ptrs, npts, ch.n, FULL, dev, top, res, stream)
+    stream.sync()
+    got = res.download((G, 2, ch.rows, ch.n))
+    digits = oc.modup(ct[1], top)
+    want = oc.cts_fused(ct[None], digits[None], top, B, G, pts, gals, seeds=seeds, bs=bs, enc=FULL)[0]
+    rs = ext_rows(ch, top)
+    for j in range(G):
+        assert (got[j][:, rs] == want[j][:, rs]).all(), j
 
 
 # ----------------------------------------------------------------------------------------------- table entries

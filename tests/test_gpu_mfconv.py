@@ -1,8 +1,8 @@
 """The conversions on the matrix cores (mfconv.hip) against the same context's launches through the kernel table alone
 (bconv, then the transforms), word for word: one to 17 sources (padded to 8, 16 and 20, one more in the exact
 conversion), targets that leave a last run of one to four, every number of targets per workgroup (1, 2, 4, 8: PCX_CC_TPW
-forces the form; 0: the context's own choice of form and number), every ring degree, 28- to 31-bit primes, and ciphertexts of words at the ends of their range
-(0, p - 1), where a digit sum that overflowed would show. Each test prints its case before the GPU runs."""
+forces the form; 0: the context's own choice of form and number), every ring degree, 28- to 31-bit primes, and ciphertexts
+of words at the ends of their range (0, p - 1). Each test prints its case before the GPU runs."""
 import sys
 
 import numpy as np
