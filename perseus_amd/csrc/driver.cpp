@@ -821,30 +821,35 @@ int mfc_shape(const pcx_ctx* c, const BconvArgs& b) {
     if (c->cc_tpw > 0) return c->cc_tpw > 2 ? (c->cc_tpw + 3) / 4 * 4 : c->cc_tpw;
     return mfc_wgs(c, b, 8) >= 3000 ? 8 : mfc_wgs(c, b, 4) >= 160 ? 4 : 2;
 }
-// Whether conversion b of plan p runs on the matrix cores: by sources, N and waves, from each call site timed both ways
-// (5 to 16 sources, N = 2^12 to 2^16, 1 to 26 keys or products, one box; us by which the matrix form is the shorter):
+// Whether conversion b of plan p runs on the matrix cores: by call site, sources, N and waves, each site timed both ways (5 to
+// 16 sources, N = 2^12 to 2^16, 1 to 26 keys or products, one box; us by which the matrix form is the shorter):
 //  Up to 4 sources the butterflies' forms sum in registers as fast.
 //  N <= 2^13: above 8 sources until the launch fills the chip (9 sources of 2^13: 80 waves +10, 800 +4, 1280 +1.6, 1600 -1,
 //   3200 -7; 16 sources: 2560 +3, 3840 -3), 7 and 8 up to 256 waves (256 +1, 320 -2, 1280 -3), 5 and 6 never (64 -1, 1280 -5).
 //   Exact conversions (bconv's extra pass on the other side): up to 256 waves (+2), above 10 sources 512 (+1, 1280 -2).
-//  N = 2^14: above 8 sources (+4 to +17); 7 and 8 up to 512 waves (+1) and from 1920 on (+2; 640 to 1280 -1 to -2); 5 and 6
-//   from 2560 on (+1; 768 -3). N = 2^15: above 6 sources (+1 to +16), 5 and 6 from 1920 on (+1; 768 -3). Exact: always
-//   (+1 to +10), but for 16 sources or more below 2048 waves (1024 -4: the form of 20 sources spills).
-//  N = 2^16: always above 6 sources (+1 to +22), 5 and 6 from 800 waves on (+2 to +17; 512 -2); exact always (+1 to +25).
-bool mfc_pays(int logn, int src, long waves, bool exact) {
+//  N = 2^14: above 8 sources (+4 to +17). ModUp: 8 (+1), 7 up to 512 waves (+1; 2304 -1). ModDown: 7 and 8 up to 512 (+0.5),
+//   8 from 1920 on (+2; 640 to 1280 -1), 7 from 3840 (+2), 5 and 6 from 2560 (+1; 768 -3).
+//  N = 2^15: above 7 sources (+1 to +16); ModDown 5 and 6 from 1920 waves on (+1; 768 -3). ModUp 5 to 7 -3 to +1.
+//  N >= 2^14 exact: always (+1 to +25), but for 16 sources or more at 2^14 and 2^15 below 2048 waves (1024 -4: the form of 20
+//   sources spills).
+//  N = 2^16: above 6 sources (+1 to +22), 5 and 6 from 800 waves on (+2 to +17; 512 -2).
+enum class Conv { up, down, exact };
+bool mfc_pays(int logn, int src, long waves, Conv at) {
     if (src <= 4) return false;
-    if (logn <= 13) {
-        if (exact) return waves <= (src > 10 ? 512 : 256);
-        return src > 8 ? waves <= 170 * (src - 1) : src > 6 && waves <= 256;
+    if (at == Conv::exact) {
+        if (logn <= 13) return waves <= (src > 10 ? 512 : 256);
+        return logn == 16 || src < 16 || waves >= 2048;
     }
-    if (exact) return logn == 16 || src < 16 || waves >= 2048;
+    if (logn <= 13) return src > 8 ? waves <= 170 * (src - 1) : src > 6 && waves <= 256;
     if (logn == 16) return src > 6 || waves >= 800;
-    if (logn == 15) return src > 6 || waves >= 1920;
-    return src > 8 || (src > 6 ? waves <= 512 || waves >= 1920 : waves >= 2560);
+    if (logn == 15) return src > 7 || (at == Conv::down && src < 7 && waves >= 1920);
+    if (src > 8) return true;
+    if (at == Conv::up) return src == 8 || (src == 7 && waves <= 512);
+    return src > 6 ? waves <= 512 || waves >= (src == 8 ? 1920 : 3840) : waves >= 2560;
 }
-bool mfc_on(const pcx_ctx* c, const Bconv& p, const BconvArgs& b, bool exact = false) {
+bool mfc_on(const pcx_ctx* c, const Bconv& p, const BconvArgs& b, Conv at) {
     if (!mf_on(c) || p.mf_ns == 0) return false;
-    return c->cc_tpw > 0 || mfc_pays((int)c->logn, p.mf_src, mfc_wgs(c, b, 4) << (c->logn / 2) >> 5, exact);
+    return c->cc_tpw > 0 || mfc_pays((int)c->logn, p.mf_src, mfc_wgs(c, b, 4) << (c->logn / 2) >> 5, at);
 }
 // The conversion b of plan p (its first b.njobs jobs) on the matrix cores, fused into the column pass of f's rows, then f's
 // row pass and epilogue. exact: p's jobs are, b.src is the context's extended workspace
@@ -917,7 +922,7 @@ int moddown_rescale(pcx_ctx* c, void* ext, int top, void* out, const void* onto,
     f.xstride = c->ct_words();
     f.es = M.ntt.es;
     f.ess = M.ntt.es + c->rows;
-    if (mfc_on(c, M.conv, b, true) && c->cc_fused) return mfc_then_rows(c, M.conv, b, f, s, true);
+    if (mfc_on(c, M.conv, b, Conv::exact) && c->cc_fused) return mfc_then_rows(c, M.conv, b, f, s, true);
     if (cc_on(c, CC_MDR)) return conv_then_rows(c, b, f, s, 5, 6, c->kp + 2, 1);
     {
         Stage st(c, 5, s);
@@ -950,7 +955,7 @@ int modup(pcx_ctx* c, const void* ct, int top, pc_stream_t s, int K = 1) {
     b.njobs = k_jobs(c, L->mu_bconv, K);
     b.max_tgt = L->mu_bconv.max_tgt;
     NttArgs f = ntt_args(c, c->digits, L->mu_ntt, k_rows(c, L->mu_ntt, K));
-    if (mfc_on(c, L->mu_bconv, b) && cc_on(c, CC_MODUP)) return mfc_then_rows(c, L->mu_bconv, b, f, s);
+    if (mfc_on(c, L->mu_bconv, b, Conv::up) && cc_on(c, CC_MODUP)) return mfc_then_rows(c, L->mu_bconv, b, f, s);
     if (cc_on(c, CC_MODUP)) return conv_then_rows(c, b, f, s, 1, 2, c->alpha);
     {
         Stage st(c, 1, s);
@@ -1137,7 +1142,7 @@ int moddown(pcx_ctx* c, void* ext, uint32_t* conv, int m, int top, void* out, pc
     b.pr = c->pr;
     b.njobs = 2 * m;
     b.max_tgt = top + 1;
-    if (mfc_on(c, L->md_bconv, b) && (c->md_fused || cc_on(c, CC_MODDOWN)))
+    if (mfc_on(c, L->md_bconv, b, Conv::down) && (c->md_fused || cc_on(c, CC_MODDOWN)))
         return mfc_then_rows(c, L->md_bconv, b, f, s);
     if (c->md_fused) {
         // the conversion inside the NTT's column pass, then the row pass with the epilogue
