@@ -871,20 +871,25 @@ __global__ void __launch_bounds__(DBX * NDIG, 3) dot_split(KsArgs A, KeyTab T, P
 }
 
 // The fast dot's launch: a wave per digit (one digit, or resident `a`: one-wave workgroups) when the launch has fewer keys
-// than a staged workgroup's waves. Without a retry table a wave per digit pays a ChaCha12 round for each digit's few
-// rejected words where the one wave pays one for all. That shows once the SIMDs have more than a workgroup each
-// (SPLIT_REDRAW) at N <= 2^14 or with more than two keys or ciphertexts: 30-bit packed keys, one wave / wave per digit, N = 2^14: 288
-// workgroups 54.5 / 51.0 us, 1120 79.2 / 76.3, 1728 90.6 / 92.9; N = 2^16: one key, 2240 workgroups, 123.4 / 117.5, two,
-// 4480, 167.2 / 159.4, four ciphertexts, 3072, 135.0 / 138.2.
-constexpr long SPLIT_REDRAW = 1200;
-inline bool split_pays(const dim3& g) {
-    return (long)g.x * g.y * g.z <= SPLIT_REDRAW || (g.x > (1 << 14) / DCH && g.z <= 2);
+// than a staged workgroup's waves.
+//  Without a retry table a wave per digit pays a ChaCha12 round for each digit's few rejected words where the one wave pays
+//  one for all. That shows once the SIMDs have more than a workgroup each at N <= 2^14 or with more than two keys or
+//  ciphertexts: 30-bit packed keys, one wave / wave per digit, N = 2^14: 288 workgroups 54.5 / 51.0 us, 1120 79.2 / 76.3, 1728
+//  90.6 / 92.9; N = 2^16: one key, 2240 workgroups, 123.4 / 117.5, two, 4480, 167.2 / 159.4, four ciphertexts, 3072, 135.0 /
+//  138.2.
+//  Two digits of several dense keys: up to 1700 workgroups the wave per
+//  digit gains 0.5 to 2 us, above it loses 0.5 to 4 (two keys at 32 rows of N = 2^15, 2048 workgroups, 79.2 / 82.2; three at
+//  14 rows of N = 2^16, 2688, 86.9 / 88.7). Three digits, and two of one key, gain at every size measured, to 12 us.
+inline bool split_pays(const dim3& g, int ndig, bool patch, int keys) {
+    const long wgs = (long)g.x * g.y * g.z;
+    if (patch) return ndig > 2 || keys < 2 || wgs <= 1700;
+    return wgs <= 1200 || (g.x > (1 << 14) / DCH && g.z <= 2);
 }
 template <int NDIG, bool PATCH, int PK = 0, bool RES = false>
 void dot_fast_launch(dim3 grid, const KsArgs& a, const KeyTab& key, const PatchTab& P, int logn, hipStream_t st) {
     if (P.diag || a.R < KW) {
         grid.z = P.diag ? a.K : a.R * a.K;
-        if (NDIG < 2 || RES || (!PATCH && !split_pays(grid))) {
+        if (NDIG < 2 || RES || !split_pays(grid, NDIG, PATCH, P.diag ? 1 : a.R)) {
             hipLaunchKernelGGL((dot_fast<NDIG, PATCH, 1, PK, RES>), grid, dim3(DBX), 0, st, a, key, P, logn);
         } else if constexpr (NDIG >= 2 && !RES) {
             hipLaunchKernelGGL((dot_split<NDIG, PATCH, PK>), grid, dim3(DBX * NDIG), 0, st, a, key, P, logn);

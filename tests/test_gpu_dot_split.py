@@ -1,7 +1,7 @@
 """The dot of few keys (dot_split: a wave per digit, the products exchanged through LDS) against the oracle's rotations,
 word for word: two and three digits, dense keys (retry table) and packed ones at 30 and 31 bits (redrawn by the wave),
-a chain that rejects a third of the words both ways, up to three keys in one launch, and packed launches on both sides of
-the size from which one wave takes all digits. Each test prints its case before the GPU runs."""
+a chain that rejects a third of the words both ways, up to three keys in one launch, and launches on both sides of the
+sizes from which one wave takes all digits. Each test prints its case before the GPU runs."""
 import sys
 
 import numpy as np
@@ -34,6 +34,7 @@ CASES = [
     ((14, 4, 2, 2, 31), [3], 31),
     ((16, 3, 1, 3, 31), [2], 0),
     ((14, 20, 8, 2, 30), [19, 9], 30),  # 448 and 1344 workgroups, 288 and 864
+    ((15, 14, 4, 2, 30), [13], 0),      # 576 and 1728
 ]
 
 
