@@ -860,6 +860,9 @@ const PrimeConst* pcx_ctx_primes(const pcx_ctx* c); /* device table by prime id 
 /* device twiddle tables [prime id][N]: fw, fws, iw, iws, then ninv, ninvs [prime id] */
 const void* pcx_ctx_twiddle(const pcx_ctx* c, int which);
 uint64_t pcx_ctx_root(const pcx_ctx* c, int prime_id);
+/* the device bytes of the context's workspace. The rows of the summed rotations and of the stages' hoisted route
+ * (max(8 min(dnum, 3), 16) (nq + kp) N words) join it with the context's first dense, full-layout rotation keys, where
+ * the device has room for them; without them those calls regenerate the keys in their kernels (the same words) */
 size_t pcx_ctx_workspace_bytes(const pcx_ctx* c);
 /* Every launch of the context's operations through the kernel table alone, as crates/pc-gpu issues them (on != 0):
  * the ModDown conversion as the table's bconv then ntt_fwd with its epilogue, the key dots as ks_dot_key (a key

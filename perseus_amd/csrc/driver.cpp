@@ -11,8 +11,10 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstdlib>
 #include <cstring>
+#include <mutex>
 #include <new>
 #include <vector>
 
@@ -359,9 +361,11 @@ struct pcx_ctx {
     std::vector<Level> levels;
     uint32_t *coef = nullptr, *digits = nullptr, *ext = nullptr, *conv = nullptr;
     uint32_t* tmp = nullptr;  // one ciphertext: the rescale's correction rows, a product's d2 (part 1)
-    // a summed rotation's expanded `a` words (ASUM_KEYS keys of every digit and row), or a transform stage's rotations
-    // (STAGE_B extended ciphertexts)
-    uint32_t* asum = nullptr;
+    // a summed rotation's expanded `a` words (ASUM_KEYS keys of asum_digits() digits and every row), or a transform stage's
+    // rotations (STAGE_B extended ciphertexts). Allocated with the first group of rotation keys that can use it
+    // (wide_workspace); null where there is none or the device had no room: the routes that regenerate the keys run
+    std::atomic<uint32_t*> asum{nullptr};
+    std::mutex asum_mu;
     size_t ws_bytes = 0;
     // stage timing (pcx_timing): event pairs recorded around each stage's launches on the launch stream
     bool timing = false;
@@ -371,6 +375,9 @@ struct pcx_ctx {
 
     size_t row_words() const { return n; }
     size_t ct_words() const { return (size_t)2 * rows * n; }
+    // the routes over asum take at most three digits
+    int asum_digits() const { return std::min(dnum, 3); }
+    size_t asum_bytes() const { return (size_t)std::max(ASUM_KEYS * asum_digits(), STAGE_B * 2) * rows * n * 4; }
     // rows of the extended ciphertexts at ext; the rows after them hold the exact conversions' u, two per ciphertext
     size_t ext_rows() const { return (size_t)std::max(k_rot, k_max) * 2 * rows; }
     int digit(int id) const { return id < nq ? id / alpha : -1; }
@@ -969,7 +976,8 @@ int modup(pcx_ctx* c, const void* ct, int top, pc_stream_t s, int K = 1) {
 // with a retry table, full rows, nothing resident. The six ciphertexts of a C4 scoring: a rung's dots 168 us (ksum_k, each
 // ciphertext regenerating the seven keys) -> 54 us
 bool sum_pre(const pcx_ctx* c, const pcx_keys* k, const Level* L) {
-    return k->pval && !c->table_only && k->bits == 0 && k->q_top < 0 && L->ndig <= 3 && !(k->ka && k->regen < L->ndig);
+    return c->asum && k->pval && !c->table_only && k->bits == 0 && k->q_top < 0 && L->ndig <= 3 &&
+           !(k->ka && k->regen < L->ndig);
 }
 
 // the dot of keys [r0, r0 + m) of k into m extended ciphertexts at ext (crates/pc-gpu/src/ks.rs:1225-1308 dot_key);
@@ -1028,18 +1036,19 @@ int dot(pcx_ctx* c, pcx_keys* k, int r0, int m, const void* ct, int top, void* e
     Stage st(c, 3, s);
     if (pre) {
         const size_t per_key = (size_t)c->dnum * c->rows * (c->n / 1024);
-        const int most = ASUM_KEYS * c->dnum * c->rows / (L->ndig * L->nks);
+        const int most = ASUM_KEYS * c->asum_digits() * c->rows / (L->ndig * L->nks);
+        uint32_t* const asum = c->asum;
         for (int j = 0; j < m; j += most) {
             const int r = std::min(most, m - j);
             const pch::PatchTab P = {k->pidx + (size_t)(r0 + j) * per_key, k->pval, c->dnum, c->rows};
-            if (int e = pch::kska_expand((int)c->logn, k->seed + r0 + j, c->pr, &P, r, L->ndig, L->ks_rows, L->nks, c->asum, s))
+            if (int e = pch::kska_expand((int)c->logn, k->seed + r0 + j, c->pr, &P, r, L->ndig, L->ks_rows, L->nks, asum, s))
                 return e;
             KsKeyArgs h = g;
             h.ks.autok = k->autok + r0 + j;
             h.ks.R = r;
             h.key.kb = k->kb + r0 + j;
             if (j) h.ks.c0_mode |= PC_KS_ACC;
-            if (int e = pch::ks_dot_key_sum_pre((int)c->logn, &h, c->asum, s)) return e;
+            if (int e = pch::ks_dot_key_sum_pre((int)c->logn, &h, asum, s)) return e;
         }
         return 0;
     }
@@ -1264,6 +1273,23 @@ pcx_keys* keys_shell(pcx_ctx* c, int nkeys, const uint64_t* galois, int bits, in
     return k;
 }
 
+// The workspace of the summed rotations and the hoisted stages, once per context, with its first rotation keys that have a
+// retry table: a context that transforms or multiplies holds none of it. Without room for it (or with PCX_WIDE_WS=0) the
+// context runs on without: nothing but those routes uses it
+void wide_workspace(pcx_ctx* c) {
+    std::lock_guard<std::mutex> lock(c->asum_mu);
+    if (c->asum) return;
+    if (const char* e = getenv("PCX_WIDE_WS"))
+        if (atoi(e) == 0) return;
+    void* p = nullptr;
+    if (hipMalloc(&p, c->asum_bytes()) != hipSuccess) {
+        (void)hipGetLastError();
+        return;
+    }
+    c->dev.owned.push_back(p);
+    c->asum = (uint32_t*)p;
+}
+
 // The retry-value table of a dense key group (a kernel counts each chunk's rejected KSKA words, the host takes the
 // exclusive prefix, a second kernel writes the redrawn values); skipped when PCX_KS_PATCH=0
 int build_patches(pcx_ctx* c, pcx_keys* k) {
@@ -1292,6 +1318,7 @@ int build_patches(pcx_ctx* c, pcx_keys* k) {
         return e;
     if (hipDeviceSynchronize() != hipSuccess) return -1;
     k->patch_words = (cells + 1) + acc;
+    if (std::any_of(k->galois.begin(), k->galois.end(), [](uint64_t g) { return g != 1; })) wide_workspace(c);
     return 0;
 }
 
@@ -1450,9 +1477,7 @@ pcx_ctx* pcx_ctx_new_k(uint32_t log_n, const uint64_t* primes, int nq, int kp, i
     c->ext = (uint32_t*)c->dev.alloc((c->ext_rows() + 2 * k_max) * rw);
     c->conv = (uint32_t*)c->dev.alloc(next * 2 * R * rw);
     c->tmp = (uint32_t*)c->dev.alloc((size_t)k_max * 2 * R * rw);
-    const size_t wide_rows = (size_t)std::max(ASUM_KEYS * dnum, STAGE_B * 2) * R;
-    c->asum = (uint32_t*)c->dev.alloc(wide_rows * rw);
-    c->ws_bytes = (wide_rows + coef_rows + (size_t)k_max * dnum * R + 2 * next * 2 * R + 2 * k_max + (size_t)k_max * 2 * R) * rw;
+    c->ws_bytes = (coef_rows + (size_t)k_max * dnum * R + 2 * next * 2 * R + 2 * k_max + (size_t)k_max * 2 * R) * rw;
     if (c->dev.err) {
         *err = c->dev.err;
         delete c;
@@ -1523,7 +1548,7 @@ const void* pcx_ctx_twiddle(const pcx_ctx* c, int which) {
     }
 }
 uint64_t pcx_ctx_root(const pcx_ctx* c, int id) { return id >= 0 && id < c->rows ? c->roots[id] : 0; }
-size_t pcx_ctx_workspace_bytes(const pcx_ctx* c) { return c->ws_bytes; }
+size_t pcx_ctx_workspace_bytes(const pcx_ctx* c) { return c->ws_bytes + (c->asum ? c->asum_bytes() : 0); }
 
 int pcx_ctx_table_only(pcx_ctx* c, int on) {
     if (!c) return -1;
@@ -1913,9 +1938,10 @@ int pcx_cts_stage(pcx_ctx* c, pcx_keys* k, int r0, int B, int G, const void* con
     // The hoisted route where its rotations fit the workspace and the fast dot takes the keys: a key regenerated once per
     // stage, its rejected words from the retry table, where the fused kernel regenerates it per four giant steps and redraws.
     // 8 x 8 steps of C3 623 -> 355 us, 5 x 5 of N = 2^12 85 -> 37
-    if (B <= STAGE_B && npts > 0 && k->pval && k->bits == 0 && k->q_top < 0 && !c->table_only && L->ndig <= 3 &&
+    uint32_t* const rot = c->asum;
+    if (rot && B <= STAGE_B && npts > 0 && k->pval && k->bits == 0 && k->q_top < 0 && !c->table_only && L->ndig <= 3 &&
         !stage_fused(B, G, L->ndig, (long)(c->n / 512) * L->nks))
-        return pcx_cts_stage_hoisted(c, k, r0, B, G, pts, npts, ptw, enc, ct, top, c->asum, res, s);
+        return pcx_cts_stage_hoisted(c, k, r0, B, G, pts, npts, ptw, enc, ct, top, rot, res, s);
     if (B > 1)
         if (int e = modup(c, ct, top, s)) return e;
     CtsRegenArgs ra;
