@@ -364,9 +364,11 @@ __global__ void __launch_bounds__(64 * MW, 4) mf_inv_rows(NttArgs A, MfTab T, in
 //
 // Bound: small launches by their chain of reads and barriers (12 rows of N = 2^12: 5.7 us, the two passes 7.6; of 2^13 7.2
 // and 8.0), large ones by the VALU (1600 rows of N = 2^14: 62 us, the two passes 72). One row of N = 2^14 is eight tiles for
-// each of its CU's waves: 10.6 us where the two passes spread it over several CUs and take 7.8, so it takes this form
-// from ONE14_ROWS rows on.
-constexpr int ONE14_ROWS = 512;
+// each of its CU's waves: 10.6 us where the two passes spread it over several CUs and take 7.8. Up to 256 rows have a CU each
+// and up to 512 half of one, so its time is a stair of steps at those counts (one launch / two passes, forward, us: 128 rows
+// 12.4 / 11.4, 144 12.6 / 13.3, 256 13.6 / 16.9, 257 18.8 / 18.2, 320 19.9 / 18.9, 336 19.9 / 20.6, 512 21.0 / 27.0, 513
+// 27.3 / 28.2, 2560 96 / 111): it is taken for 129 to 256 rows and above 320 (one14).
+inline bool one14(int rows) { return (rows > 128 && rows <= 256) || rows > 320; }
 template <int LOGN>
 struct Mo {
     using M = Mg<LOGN>;
@@ -608,7 +610,7 @@ inline int mf_check(const NttArgs* a, const MfTab* t, bool fwd) {
 }
 // whether a whole transform of rows of N takes the one-pass form
 template <int LOGN>
-bool mf_one(int rows) { return rows > 0 && (LOGN <= 13 || rows >= ONE14_ROWS); }
+bool mf_one(int rows) { return rows > 0 && (LOGN <= 13 || one14(rows)); }
 template <int LOGN, int CAN>
 void mf_one_launch(const NttArgs& A, const MfTab& T, const RescaleArgs* R, hipStream_t st) {
     const dim3 g(A.nrows), b(64 * Mo<LOGN>::W);

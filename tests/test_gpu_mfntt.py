@@ -10,6 +10,7 @@ import numpy as np
 import pytest
 
 import perseus_amd as pa
+from perseus_amd.chains import make
 from tests import twin
 
 pytestmark = pytest.mark.gpu
@@ -53,9 +54,55 @@ def test_transforms_at_the_rule(stream, logn, bits, rows):
     transforms(stream, logn, bits, rows)
 
 
-def test_transforms_one_pass(stream):
-    """N = 2^14 in one pass: a launch of more rows than the two passes take (N = 2^12 and 2^13 always do)"""
-    transforms(stream, 14, 31, 517)
+@pytest.mark.parametrize("bits,rows", [(31, 128), (28, 129), (31, 256), (28, 257), (31, 320), (28, 321), (31, 517)])
+def test_transforms_one_pass(stream, bits, rows):
+    """N = 2^14 on both sides of the row counts that take one launch (N = 2^12 and 2^13 always do)"""
+    transforms(stream, 14, bits, rows)
+
+
+@pytest.mark.parametrize("bits,K", [(28, 4), (31, 8)])
+def test_one_pass_epilogues(stream, bits, K):
+    """N = 2^14 in one launch with each epilogue (the ModDown's subtraction, alone and added onto a ciphertext, the
+    rescale's addition after one prime and after two, whose rows are generated), 192 to 416 rows: against the kernel table"""
+    ch = make("one14", 14, 26, 7, 2, bits)
+    say(f"[mfntt] N=2^14, {bits}-bit primes, {K} ciphertexts: epilogues in one launch against the kernel table")
+    ctx = pa.Context(ch, k_rot=K, k_max=K)
+    rng = np.random.default_rng(K)
+    s = rng.integers(-1, 2, ch.n).astype(np.int8)
+    gals = [twin.rotation_galois(r, ch.n) for r in (1, 2, 3)]
+    seeds = rng.integers(0, 2**32, (3, 8), dtype=np.uint64).astype(np.uint32)
+    err = rng.integers(-3, 4, (3, ch.dnum, ch.n)).astype(np.int64)
+    keys = pa.Keys(ctx, gals, seeds=seeds, secret=s, errors=err, bits=0)
+    relin = pa.Keys(ctx, [1], seeds=seeds[:1], secret=s, errors=err[:1], bits=0, relin=True)
+    top, ct = 25, np.zeros((K, 2, ch.rows, ch.n), np.uint32)
+    for t in range(ch.rows):
+        ct[:, :, t] = rng.integers(0, ch.primes[t], (K, 2, ch.n))
+    x, out, tmp = pa.DevBuf.from_array(ct), ctx.ct_buf(K), ctx.ct_buf(K)
+    ctx.conv_fusion(0)  # conversions apart from the transforms, which then run whole
+
+    def moddown():
+        tmp.upload(ct, stream)  # its INTT runs in place
+        ctx.moddown_k(tmp, top, out, K, stream)
+
+    ops = [
+        ("ModDown", top + 1, moddown),
+        ("ModDown onto", top + 1, lambda: ctx.rotate_and_sum(keys, x, top, 1, 4, out, tmp, stream, radix_bits=2, K=K)),
+        ("rescale by one", top, lambda: ctx.rescale(x, top, 1, out, stream, K=K)),
+        ("rescale by two", top - 1, lambda: ctx.rescale(x, top, 2, out, stream, K=K)),
+        ("product, rescaled", top - 1, lambda: ctx.mul_relin_rescale(relin, x, x, top, out, stream, K=4)),
+    ]
+    for name, limbs, f in ops:
+        say(f"[mfntt]   {name}")
+        got = []
+        for table in (False, True):
+            ctx.table_only(table)
+            ctx.conv_fusion(0)
+            out.zero()
+            f()
+            stream.sync()
+            got.append(out.download((K, 2, ch.rows, ch.n))[:, :, :limbs])
+        ctx.table_only(False)
+        assert (got[0] == got[1]).all(), name
 
 
 def transforms(stream, logn, bits, rows=0):
