@@ -1,11 +1,12 @@
-"""The conversions streamed into the forward NTT's column pass (pch::conv_cols: the ModUp of every digit, the ModDown
-over more special primes than the register-held fused form takes, and the ModDown-rescale's exact conversion of
-kp + 2 sources) against the plan's bconv then ntt_fwd, word for word, through the C-ABI: the same context runs each
-operation with pcx_ctx_conv_fusion on (7) and off (0). Chains: C5 (30-bit primes, Harvey butterflies, 16 special
-primes, digits of 16 limbs), C3 (31-bit primes: non-lazy butterflies, and products whose sums fold to a residue
-every 4 sources), and N = 2^12 / 2^14 chains of 16 special primes (other column-pass shapes); tops that leave a
-partial digit, a single limb, and K = 2 ciphertexts. The fused path against the oracle is covered by the rotation,
-product and bootstrap tests, which run it by default."""
+"""The conversions streamed into the forward NTT's column pass (the ModUp of every digit, the ModDown over more special
+primes than the register-held fused form takes, and the ModDown-rescale's exact conversion of kp + 2 sources) against the
+plan's bconv then ntt_fwd, word for word, through the C-ABI: the same context runs each operation with
+pcx_ctx_conv_fusion on (7) and off (0). Chains: C5 (30-bit primes, 16 special primes, digits of 16 limbs), C3 (31-bit
+primes), and N = 2^12 / 2^14 chains of 16 special primes (other column-pass shapes); tops that leave a partial digit, a
+single limb, and K = 2 ciphertexts. Contexts of these chains stream on the matrix cores where that form is taken; with a
+27-bit prime as the last special one ("_27") they run the butterflies' form at every size: pch::conv_cols, fast and exact,
+with Harvey butterflies at 30 bits, and at 31 bits non-lazy ones and sums that fold to a residue every 4 sources. The
+streamed paths against the oracle are covered by the rotation, product and bootstrap tests, which run them by default."""
 import sys
 
 import numpy as np
@@ -43,12 +44,16 @@ _SETUP = {}
 
 def setup(name):
     if name not in _SETUP:
-        if name == "t12":
+        base = name.removesuffix("_27")
+        if base == "t12":
             ch = make("t12", 12, 20, 16, 3, 30)
-        elif name == "t14":
+        elif base == "t14":
             ch = make("t14", 14, 26, 16, 3, 30)
         else:
-            ch = pa.preset(name)
+            ch = pa.preset(base)
+        if name != base:
+            small = twin.descending_primes(27, 2 << ch.logn, 1)
+            ch = pa.Chain(name, ch.logn, ch.q, list(ch.p[:-1]) + small, ch.dnum)
         ctx = pa.Context(ch, k_rot=2, k_max=2)
         rng = np.random.default_rng(len(name) * 7 + ch.logn)
         s = rng.integers(-1, 2, ch.n).astype(np.int8)
@@ -72,9 +77,11 @@ def both(ctx, fn):
     return a, b
 
 
+@pytest.mark.parametrize("form", ["", "_27"])
 @pytest.mark.parametrize("name,tops", [("c5", [46, 31, 16, 0]), ("c3", [29, 20, 9]), ("t12", [19, 8, 2]),
                                        ("t14", [25, 15])])
-def test_rotation_fused_equals_unfused(stream, name, tops):
+def test_rotation_fused_equals_unfused(stream, name, tops, form):
+    name += form
     ch, ctx, keys = setup(name)
     rng = np.random.default_rng(11)
     for top in tops:
@@ -92,10 +99,12 @@ def test_rotation_fused_equals_unfused(stream, name, tops):
         assert (a[:, : top + 1] == b[:, : top + 1]).all()
 
 
-@pytest.mark.parametrize("name,tops", [("c5", [46, 33, 17, 2]), ("c3", [29, 12, 2]), ("t12", [19, 5])])
-def test_product_rescale_fused_equals_unfused(stream, name, tops):
+@pytest.mark.parametrize("form", ["", "_27"])
+@pytest.mark.parametrize("name,tops", [("c5", [46, 33, 17, 2]), ("c3", [29, 12, 2]), ("t12", [19, 5]), ("t14", [25, 9])])
+def test_product_rescale_fused_equals_unfused(stream, name, tops, form):
     """the relinearized product and its two-prime rescale in one ModDown (the exact conversion of kp + 2 sources),
     K = 1 and K = 2 pairs"""
+    name += form
     ch, ctx, keys = setup(name)
     rng = np.random.default_rng(12)
     for top in tops:
@@ -115,9 +124,10 @@ def test_product_rescale_fused_equals_unfused(stream, name, tops):
             assert (x[:, :, : top - 1] == y[:, :, : top - 1]).all()
 
 
-def test_modup_digits_fused_equal_unfused(stream):
+@pytest.mark.parametrize("form", ["", "_27"])
+def test_modup_digits_fused_equal_unfused(stream, form):
     """the ModUp alone: every digit's rows of the workspace, C5 at a top inside the third digit"""
-    ch, ctx, keys = setup("c5")
+    ch, ctx, keys = setup("c5" + form)
     rng = np.random.default_rng(13)
     top = 40
     x = pa.DevBuf.from_array(random_ct(ch, top, rng)[0])
