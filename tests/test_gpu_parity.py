@@ -157,12 +157,12 @@ def test_dot_and_moddown(stream, name, top, bits):
 
 def test_moddown_table_path(stream, monkeypatch):
     """ModDown through the kernel table's separate stages (INTT, bconv, NTT with epilogue 1), the path the driver takes
-    when the conversion cannot be fused into the NTT column pass (more than 6 special primes): same words as the fused
-    path and the oracle."""
+    when no conversion is fused into the NTT column pass: same words as the fused path and the oracle."""
     say("[moddown table path] c3 top=29")
     monkeypatch.setenv("PCX_MD_FUSED", "0")
     ch = pa.preset("c3")
     ctx = pa.Context(ch, k_rot=1)
+    ctx.conv_fusion(0)
     _, _, oc = contexts("c3")
     top = len(ch.q) - 1
     rng = np.random.default_rng(11)
