@@ -9,6 +9,9 @@
 // 128 sum W and a bias that keeps every S_i non-negative are the accumulator's initial value. With |b - 128| and |w|
 // at most 128, |sum| <= 64 2^14 = 2^20, so S_i < 2^21 + 2^8 and the value is below 2^46: one quotient estimate reduces
 // it to r < 1.13 p + 2^29.01 (mf_reduce). The words between steps are any 32-bit words, so no step needs a correction.
+// A conversion of 17 to 20 sources has depth 80: |sum| <= 80 2^14 = 1.25 2^20 under a bias of 2^21, so S_i < 3.25 2^20 + 2^8,
+// S_2 + S_3 2^8 and S_0 + S_1 2^8 are below 257 (3.25 2^20 + 2^8) < 2^29.71, and the estimate is low by less than 1 +
+// 2^29.71 / 2^32 < 1.21: r < 1.21 p + 2^29.71, below 2^32 for p < 2^31.
 //
 // A radix-rho step of the transform at a level of m blocks takes block i's words x_k (k < rho, N / (rho m) apart) to
 // their values at the rho roots: out_c = sum_k (x_k eta^k) omega^(k brev(c)), eta = fw[(rho / 2)(m + i)], omega =
@@ -61,7 +64,7 @@ struct MfPrime {
     }
 };
 
-// S_0 + S_1 2^8 + S_2 2^16 + S_3 2^24 as a word r == it (mod p). With hi = S_2 + S_3 2^8 < 2^29.01, the quotient q =
+// S_0 + S_1 2^8 + S_2 2^16 + S_3 2^24 as a word r == it (mod p), at depth 64. With hi = S_2 + S_3 2^8 < 2^29.01, the quotient q =
 // floor(hi mu / 2^32) of hi 2^16 by p is low by less than 1.13, so hi 2^16 - q p < 1.13 p and r < 1.13 p + lo, lo < 2^29.01:
 // below 2^32 for every p < 2^31.
 template <int SH>

@@ -72,7 +72,7 @@ __device__ __forceinline__ void quarter_transpose(uint32_t& a0, uint32_t& a1, ui
     const v2u v = __builtin_amdgcn_permlane16_swap(x.y, y.y, false, false);
     a0 = u.x, a1 = u.y, a2 = v.x, a3 = v.y;
 }
-// mf_reduce with a prime of the lane's own (np = 2^32 - p)
+// mf_reduce with a prime of the lane's own (np = 2^32 - p); also at the 20 sources' depth of 80 (mf.h: r < 1.21 p + 2^29.71)
 __device__ __forceinline__ uint32_t mf_reduce_lane(const v4i& s, uint32_t np, uint32_t mu) {
     const uint32_t lo = ((uint32_t)s.y << 8) + (uint32_t)s.x, hi = ((uint32_t)s.w << 8) + (uint32_t)s.z;
     return __umulhi(hi, mu) * np + lshl_add<16>(hi, lo);  // two instructions: v_mad_u64_u32's pairs spill here
@@ -342,7 +342,8 @@ void mf_conv_digits(const uint64_t* w, int n, int nt, const uint64_t* p, int ns,
                 for (int k = 0; k < 4; ++k) blk[((16 * (ii / per) + 4 * t + k) * per + ii % per) * 4 + a] = d[k];
             }
         }
-        // sum_i c_i 2^(8i) == 128 sum W (mod p) with c_i = B + d_i, B >= the largest |sum| of a digit's products
+        // sum_i c_i 2^(8i) == 128 sum W (mod p) with c_i = B + d_i, B >= the largest |sum| of a digit's products (2^20 at depth
+        // 64, 1.25 2^20 at 80)
         const uint64_t need = (sum * 128 + p[t] - B * ones % p[t]) % p[t];
         for (int k = 0; k < 4; ++k) out[ns * 16 + 4 * t + k] = (uint32_t)(B + ((need >> (8 * k)) & 255));
     }
