@@ -185,7 +185,9 @@ __global__ void __launch_bounds__(Mc<LOGN>::TH, LOGN < 14 ? 3 : 4) mf_conv_cols(
                             d = __builtin_amdgcn_mfma_i32_16x16x64_i8(a0, b, d, 0, 0, 0);
                         }
                         if constexpr (NS == 20) {
-                            // (a 16x16x32 MFMA onto the 16x16x64's result gave wrong words)
+                            // not the 16x16x32 form: the compiler issues it right behind the 16x16x64 whose result it
+                            // accumulates onto, and half its words then miss that result (alone, 128 of 256 words
+                            // wrong back to back, none with wait states between or with the two sums added)
                             const v4i b = {(int)(s[4] ^ MF_FLIP), 0, 0, 0};
                             d = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, b, d, 0, 0, 0);
                         }
