@@ -750,16 +750,20 @@ NttArgs ntt_args(const pcx_ctx* c, void* base, const Rows& r, int nrows) {
 // The transforms: on the matrix cores (mf.h), or through the kernel table's butterflies where a caller asks for the
 // table alone, for the one-pass form, where the context's primes are below the matrix passes' range, or where they are faster
 bool mf_on(const pcx_ctx* c) { return c->mf.can > 0 && !c->table_only; }
-// Where the butterflies stay the faster whole transform (medians of alternating runs on one box, butterflies / matrix):
-//  N = 2^15 past the last-level cache's 256 MB: primes below 2^30 from 2048 rows on (forward 2048 rows 192.7 / 197.3 us,
-//   2560 273 / 302, 4096 449 / 476, inverse 2560 278 / 288; at 1792 rows 161 / 153), 31-bit ones forward above 2112 (2112
-//   rows +1.5% for the matrix form, 2176 -6%, 2560 280 / 304); N = 2^16 gains at every size (2560 rows 576 / 567).
+// Where the butterflies stay the faster whole transform (medians of alternating runs on one box over three buffers in turn,
+// as fresh inputs come, butterflies / matrix, us):
+//  N = 2^15 forward, whose column pass reads its rows from memory once the inputs no longer lie in the last-level cache:
+//   primes below 2^30 from 672 rows on (640 rows 65.9 / 63.5, 700 73.6 / 77.0, 1024 105.9 / 117.8, 2560 282.9 / 304.3),
+//   31-bit ones from 784 (768 rows 84.6 / 84.3, 800 87.3 / 89.8, 2560 289.6 / 304.3). (One buffer over and over, the matrix
+//   form keeps 4 to 14% up to 1792 rows.) N = 2^16 gains at nearly every size (1600 rows +2%, 400 +1%, 320 +12%).
 //  The inverse of few rows of primes below 2^30, whose lazy butterflies are the shorter chain: N = 2^14 12 rows 7.98 / 8.36,
-//   40 rows -2%, 48 even; 2^15 12 rows 8.59 / 8.88, 160 rows -3%, 200 +2%; 2^16 12 rows 9.06 / 9.31, 24 even. At N = 2^12
-//   and 2^13 the one launch always pays (one row 6.5 / 5.2 and 7.3 / 6.7).
+//   40 rows -2%, 48 even; 2^15 12 rows 8.59 / 8.88, 160 20.9 / 21.7, 256 31.3 / 31.5, 400 46.3 / 44.4; 2^16 12 rows 9.06 /
+//   9.31, 24 even; and of many of N = 2^15 (2048 rows +4%, 2100 -1%, 2560 286.4 / 293.4).
+//  At N = 2^12 and 2^13 the one launch always pays (one row 6.5 / 5.2 and 7.3 / 6.7).
 bool mf_ntt_pays(const pcx_ctx* c, int rows, bool fwd) {
-    if (c->logn == 15 && (c->lazy ? rows >= 2048 : fwd && rows > 2112)) return false;
-    return fwd || !c->lazy || c->logn < 14 || rows > (c->logn == 14 ? 40 : c->logn == 15 ? 160 : 16);
+    if (c->logn == 15 && fwd) return rows < (c->lazy ? 672 : 784);
+    if (fwd || !c->lazy || c->logn < 14) return true;
+    return c->logn == 15 ? rows > 256 && rows <= 2080 : rows > (c->logn == 14 ? 40 : 16);
 }
 bool mf_ntt_on(const pcx_ctx* c, int rows, bool fwd) {
     return mf_on(c) && !pch::ntt_one_pass((int)c->logn, rows) && mf_ntt_pays(c, rows, fwd);

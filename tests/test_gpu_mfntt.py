@@ -45,10 +45,10 @@ def test_transforms(stream, logn, bits):
 
 
 # both sides of the rows from which, or up to which, the butterflies are taken (driver.cpp mf_ntt_pays): the inverse of few
-# rows of primes below 2^30, N = 2^15 past the last-level cache
+# rows of primes below 2^30 and of many of N = 2^15, the forward of N = 2^15 past the last-level cache
 @pytest.mark.parametrize("logn,bits,rows", [
-    (14, 28, 40), (14, 30, 41), (15, 28, 160), (15, 30, 161), (16, 28, 16), (16, 30, 17),
-    (15, 30, 2047), (15, 28, 2048), (15, 31, 2112), (15, 31, 2113),
+    (14, 28, 40), (14, 30, 41), (15, 28, 256), (15, 30, 257), (16, 28, 16), (16, 30, 17),
+    (15, 30, 671), (15, 28, 672), (15, 31, 783), (15, 31, 784), (15, 28, 2080), (15, 30, 2081),
 ])
 def test_transforms_at_the_rule(stream, logn, bits, rows):
     transforms(stream, logn, bits, rows)
