@@ -47,9 +47,9 @@ KERNELS = {
             "dot_fast<3, true, 4, 0, false>: key inner product of all 26 keys, a regenerated by ChaCha12"),
     "md_ntt": ("pch::ntt::mf_fwd_", "mf_fwd_rows<epilogue 1>: ModDown NTT row pass, (x - conv) P^-1"),
     "md_intt": ("pch::ntt::mf_inv_", "mf_inv_rows + mf_inv_cols: ModDown INTT of the P rows"),
-    "md_bconv": ("pch::bconv::bconv_k", "bconv_k: ModDown P -> Q conversion"),
+    "md_bconv": ("pch::ntt::mf_conv_cols<16, 8>", "mf_conv_cols<16, 8>: ModDown P -> Q conversion and NTT column pass"),
     "modup_intt": ("pch::ntt::mf_inv_", "mf_inv_rows + mf_inv_cols: ModUp INTT"),
-    "modup_bconv": ("pch::bconv::bconv_k", "bconv_k: ModUp conversion"),
+    "modup_bconv": ("pch::ntt::mf_conv_cols<16, 16>", "mf_conv_cols<16, 16>: ModUp conversion and NTT column pass"),
     "modup_ntt": ("pch::ntt::mf_fwd_", "mf_fwd_rows: ModUp NTT row pass"),
 }
 

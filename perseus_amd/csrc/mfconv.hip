@@ -14,9 +14,9 @@
 // mf_fwd_cols takes a row. The prime's two matrices (8 KB) and twiddles go through LDS, loaded once per workgroup and
 // target, a target ahead.
 //
-// Bound: latency. 26 ModDowns of C3 (6 sources, 1560 target rows) take 196 us where their 0.49 GB of traffic takes about
-// 95: 54% VALU busy (31 instructions per word, 10 of them beside the arithmetic), 24% LDS, 20% matrix core, two
-// workgroups per CU whose waves wait on four chained reads at their start and on a barrier per target. The butterflies'
+// Bound: latency. 26 ModDowns of C3 (6 sources, 1560 target rows) take 196 us where their 0.58 GB of traffic takes about
+// 104: 48% VALU busy (30 instructions per word, 10 of them beside the arithmetic), 19% matrix core, no LDS bank conflicts,
+// two workgroups per CU whose waves wait on four chained reads at their start and on a barrier per target. The butterflies'
 // form took 265 us (md_conv_cols_k); C3's ModUp 33 -> 21 us, C5's ModUp of four ciphertexts 100 -> 77 us, the exact
 // conversion of 8 x 33 rows (bconv_k, then the column pass) 150 -> 74 us. Sources held in registers over all of a
 // workgroup's targets (184-254 registers, one workgroup per CU) took 235-340 us for the first.
