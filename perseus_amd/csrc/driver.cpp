@@ -756,24 +756,29 @@ bool mf_on(const pcx_ctx* c) { return c->mf.can > 0 && !c->table_only; }
 //   primes below 2^30 from 672 rows on (640 rows 65.9 / 63.5, 700 73.6 / 77.0, 1024 105.9 / 117.8, 2560 282.9 / 304.3),
 //   31-bit ones from 784 (768 rows 84.6 / 84.3, 800 87.3 / 89.8, 2560 289.6 / 304.3). (One buffer over and over, the matrix
 //   form keeps 4 to 14% up to 1792 rows.) N = 2^16 gains at nearly every size (1600 rows +2%, 400 +1%, 320 +12%).
-//  The inverse of few rows of primes below 2^30, whose lazy butterflies are the shorter chain: N = 2^14 12 rows 7.98 / 8.36,
-//   40 rows -2%, 48 even; 2^15 12 rows 8.59 / 8.88, 160 20.9 / 21.7, 256 31.3 / 31.5, 400 46.3 / 44.4; 2^16 12 rows 9.06 /
-//   9.31, 24 even; and of many of N = 2^15 (2048 rows +4%, 2100 -1%, 2560 286.4 / 293.4).
+//  The inverse of few rows of primes below 2^30, whose lazy butterflies are the shorter chain. A caller's own transform
+//   (alone): N = 2^14 12 rows 7.98 / 8.36, 40 rows -2%, 48 even; 2^15 12 rows 8.59 / 8.88, 160 20.9 / 21.7, 256 31.3 / 31.5,
+//   400 46.3 / 44.4; 2^16 12 rows 9.06 / 9.31, 24 even; and many of N = 2^15 (2048 rows +4%, 2100 -1%, 2560 286.4 / 293.4).
+//   Between a key switch's other launches the matrix form pays sooner: a rotation by butterflies' inverses at N = 2^14 -1.1 us
+//   (6 and 12 rows), -0.5 (30), at 2^15 -0.3 (12), +0.7 (30), +1.7 (60), at 2^16 -0.2 (6), +0.7 (12), +1.5 (30).
 //  At N = 2^12 and 2^13 the one launch always pays (one row 6.5 / 5.2 and 7.3 / 6.7).
-bool mf_ntt_pays(const pcx_ctx* c, int rows, bool fwd) {
+bool mf_ntt_pays(const pcx_ctx* c, int rows, bool fwd, bool alone) {
     if (c->logn == 15 && fwd) return rows < (c->lazy ? 672 : 784);
     if (fwd || !c->lazy || c->logn < 14) return true;
-    return c->logn == 15 ? rows > 256 && rows <= 2080 : rows > (c->logn == 14 ? 40 : 16);
+    if (c->logn == 14) return rows > 40;
+    if (c->logn == 15) return rows > (alone ? 256 : 16) && rows <= 2080;
+    return rows > (alone ? 16 : 6);
 }
-bool mf_ntt_on(const pcx_ctx* c, int rows, bool fwd) {
-    return mf_on(c) && !pch::ntt_one_pass((int)c->logn, rows) && mf_ntt_pays(c, rows, fwd);
+bool mf_ntt_on(const pcx_ctx* c, int rows, bool fwd, bool alone) {
+    return mf_on(c) && !pch::ntt_one_pass((int)c->logn, rows) && mf_ntt_pays(c, rows, fwd, alone);
 }
-int nt_fwd(const pcx_ctx* c, const NttArgs* a, pc_stream_t s) {
-    if (!mf_ntt_on(c, a->nrows, true)) return c->tab->ntt_fwd(a, s);
+// alone: a caller's transform (pcx_ntt), not one of an operation's launches
+int nt_fwd(const pcx_ctx* c, const NttArgs* a, pc_stream_t s, bool alone = false) {
+    if (!mf_ntt_on(c, a->nrows, true, alone)) return c->tab->ntt_fwd(a, s);
     return pch::mf_ntt_fwd((int)c->logn, a, &c->mf, s);
 }
-int nt_inv(const pcx_ctx* c, const NttArgs* a, pc_stream_t s) {
-    if (!mf_ntt_on(c, a->nrows, false)) return c->tab->ntt_inv(a, s);
+int nt_inv(const pcx_ctx* c, const NttArgs* a, pc_stream_t s, bool alone = false) {
+    if (!mf_ntt_on(c, a->nrows, false, alone)) return c->tab->ntt_inv(a, s);
     return pch::mf_ntt_inv((int)c->logn, a, &c->mf, s);
 }
 int nt_fwd_rows(const pcx_ctx* c, const NttArgs* a, pc_stream_t s) {
@@ -1599,7 +1604,7 @@ int pcx_ntt_one_pass_min(int rows) { return pch::ntt_one_pass_min(rows); }
 int pcx_ntt(pcx_ctx* c, int dir, void* base, const pcx_rows* rows, pc_stream_t s) {
     if (!c || !rows || (dir != 1 && dir != -1)) return -1;
     NttArgs a = ntt_args(c, base, rows->r, rows->r.n);
-    return dir == 1 ? nt_fwd(c, &a, s) : nt_inv(c, &a, s);
+    return dir == 1 ? nt_fwd(c, &a, s, true) : nt_inv(c, &a, s, true);
 }
 
 // A key group from host b ([ndig][srows][N] per key, dense words) and seeds, banded at q_top (nq - 1: full rows)
